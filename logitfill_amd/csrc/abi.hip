@@ -13,6 +13,7 @@ int launch_pack_pages_multi(const lf_packed_layer* layers_dev, const lf_packed_l
                             int src_dtype, const int32_t* jobs, int n_jobs, hipStream_t stream);
 int launch_decode_valu(const DecodeParams& p, hipStream_t stream);
 int launch_decode_mfma(const DecodeParams& p, hipStream_t stream, bool* handled);
+int launch_decode_tiled(const DecodeParams& p, hipStream_t stream, bool* handled);
 int launch_dequantize(const lf_packed_layer& L, int b, int tokens, float* k_out, float* v_out,
                       hipStream_t stream);
 int launch_dense_decode(const void* query, const void* k, const void* v, int batch, int n_q, int n_kv,
@@ -123,6 +124,8 @@ int32_t decode_checked(const lf_packed_layer* layer, const lf_decode_args* args,
         bool handled = false;
         const int r = launch_decode_mfma(p, s, &handled);
         if (handled || A.kernel == 2) return handled ? r : LF_E_UNSUPPORTED;
+        const int rt = launch_decode_tiled(p, s, &handled);
+        if (handled) return rt;
     }
     return launch_decode_valu(p, s);
 }

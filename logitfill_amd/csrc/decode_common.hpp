@@ -118,6 +118,67 @@ __device__ __forceinline__ i32x2 prefetch_args_rec2(uint32_t off) {
 #undef LF_ARG_LINES6
 #undef LF_ARG_LINE
 
+// a[t] for a run-time t in 0..3 (or 0..2) of a kernel-argument array, through selects over
+// SGPR copies.  A dynamic index into the argument block would copy it to scratch memory; a plain
+// select chain with a per-lane t the compiler turns into a select of *addresses* and one vector
+// load from the argument block per lane -- a memory round trip each, in the prologue's
+// dependent chain.  The empty asm pins the four values in SGPRs (scalar loads, already
+// prefetched), so the select is four VALU ops.
+template <class T>
+__device__ __forceinline__ T sel4(const T (&a)[4], int t) {
+    T a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
+    asm volatile("" : "+s"(a0), "+s"(a1), "+s"(a2), "+s"(a3));
+    return t == 0 ? a0 : t == 1 ? a1 : t == 2 ? a2 : a3;
+}
+
+typedef __attribute__((address_space(3))) void lds_void;
+
+// LDS-DMA: each lane's 16 bytes at ``g`` land at lds + 16 * lane.  Issued through asm so the
+// compiler does not order every later LDS read behind it (it cannot tell the buffers apart and
+// would wait for all DMA in flight); the waits are explicit instead.  The compiler writes M0 just
+// before the asm; an LDS-DMA instruction needs one wait state after an SALU write of M0, hence
+// the s_nop.  The load carries the non-temporal (streaming) cache hint: the L2 evicts those
+// lines first and keeps what the launch reads again (its instructions, arguments, q) and the
+// partials the reduce kernel reads next (c2: 71.7 -> 70.6 us per layer-step, c1 21.5 -> 20.9 in
+// a same-box A/B; several row tiles of one kv head still find the pages in L2).
+__device__ __forceinline__ uint32_t lds_addr(unsigned char* p) {
+    return __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)p)));
+}
+__device__ __forceinline__ void dma16(const unsigned char* g, uint32_t lds) {
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "{m0}"(lds) : "memory");
+}
+
+// Max / sum of x over the four 16-lane rows (lanes l, l ^ 16, l ^ 32, l ^ 48), in every lane:
+// v_permlane16_swap pairs rows (0, 1), (2, 3); v_permlane32_swap pairs the wave halves.  Both
+// swapped registers pass through an empty asm: this compiler otherwise takes the two results
+// of a swap to be equal and drops the second.
+template <bool Half32>
+__device__ __forceinline__ void swap_rows(float x, float& a, float& b) {
+    const int xi = __builtin_bit_cast(int, x);
+    const auto r = Half32 ? __builtin_amdgcn_permlane32_swap(xi, xi, false, false)
+                          : __builtin_amdgcn_permlane16_swap(xi, xi, false, false);
+    int r0 = r[0], r1 = r[1];
+    asm volatile("" : "+v"(r0), "+v"(r1));
+    a = __builtin_bit_cast(float, r0);
+    b = __builtin_bit_cast(float, r1);
+}
+__device__ __forceinline__ float halves_sum(float x) {
+    float a, b;
+    swap_rows<true>(x, a, b);
+    return a + b;
+}
+__device__ __forceinline__ float rows_sum(float x) {
+    float a, b;
+    swap_rows<false>(x, a, b);
+    return halves_sum(a + b);
+}
+__device__ __forceinline__ float rows_max(float x) {
+    float a, b;
+    swap_rows<false>(x, a, b);
+    swap_rows<true>(fmaxf(a, b), a, b);
+    return fmaxf(a, b);
+}
+
 // The commit folded into the decode (lf_decode_args.commit_new): the workgroup that owns
 // sequence b's residual for kv head h (row tile 0) copies the new rows into the tail buffer at
 // the device-side tail length every decode workgroup reads; nothing in the launch reads those

@@ -51,7 +51,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
@@ -116,34 +115,6 @@ __device__ __forceinline__ void dma_barrier(int n) {
 // s_waitcnt lgkmcnt(0); s_barrier: every wave's LDS operations are done; DMA in flight stays
 // in flight (__syncthreads would also wait for it).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// a[t] for a run-time t in 0..3 (or 0..2) of a kernel-argument array, through selects over
-// SGPR copies.  A dynamic index into the argument block would copy it to scratch memory; a plain
-// select chain with a per-lane t the compiler turns into a select of *addresses* and one vector
-// load from the argument block per lane -- a memory round trip each, in the prologue's
-// dependent chain.  The empty asm pins the four values in SGPRs (scalar loads, already
-// prefetched), so the select is four VALU ops.
-template <class T>
-__device__ __forceinline__ T sel4(const T (&a)[4], int t) {
-    T a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
-    asm volatile("" : "+s"(a0), "+s"(a1), "+s"(a2), "+s"(a3));
-    return t == 0 ? a0 : t == 1 ? a1 : t == 2 ? a2 : a3;
-}
-
-// LDS-DMA: each lane's 16 bytes at ``g`` land at lds + 16 * lane.  Issued through asm so the
-// compiler does not order every later LDS read behind it (it cannot tell the buffers apart and
-// would wait for all DMA in flight); the waits are explicit instead.  The compiler writes M0 just
-// before the asm; an LDS-DMA instruction needs one wait state after an SALU write of M0, hence
-// the s_nop.  The load carries the non-temporal (streaming) cache hint: the L2 evicts those
-// lines first and keeps what the launch reads again (its instructions, arguments, q) and the
-// partials the reduce kernel reads next (c2: 71.7 -> 70.6 us per layer-step, c1 21.5 -> 20.9 in
-// a same-box A/B; several row tiles of one kv head still find the pages in L2).
-__device__ __forceinline__ uint32_t lds_addr(unsigned char* p) {
-    return __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)p)));
-}
-__device__ __forceinline__ void dma16(const unsigned char* g, uint32_t lds) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "{m0}"(lds) : "memory");
-}
 
 // Bit patterns of the exponent-field code unpack, held in VGPRs: with register operands the
 // compiler selects (x & mask) | bits as one v_and_or_b32 (VOP3 takes no literal), and the
@@ -292,37 +263,6 @@ __device__ __forceinline__ float qs_math(const QsRegs& r, half8* qs_hi, half8* q
     *qs_hi = hi;
     *qs_lo = lo;
     return bsum;
-}
-
-// Max / sum of x over the four 16-lane rows (lanes l, l ^ 16, l ^ 32, l ^ 48), in every lane:
-// v_permlane16_swap pairs rows (0, 1), (2, 3); v_permlane32_swap pairs the wave halves.  Both
-// swapped registers pass through an empty asm: this compiler otherwise takes the two results
-// of a swap to be equal and drops the second.
-template <bool Half32>
-__device__ __forceinline__ void swap_rows(float x, float& a, float& b) {
-    const int xi = __builtin_bit_cast(int, x);
-    const auto r = Half32 ? __builtin_amdgcn_permlane32_swap(xi, xi, false, false)
-                          : __builtin_amdgcn_permlane16_swap(xi, xi, false, false);
-    int r0 = r[0], r1 = r[1];
-    asm volatile("" : "+v"(r0), "+v"(r1));
-    a = __builtin_bit_cast(float, r0);
-    b = __builtin_bit_cast(float, r1);
-}
-__device__ __forceinline__ float halves_sum(float x) {
-    float a, b;
-    swap_rows<true>(x, a, b);
-    return a + b;
-}
-__device__ __forceinline__ float rows_sum(float x) {
-    float a, b;
-    swap_rows<false>(x, a, b);
-    return halves_sum(a + b);
-}
-__device__ __forceinline__ float rows_max(float x) {
-    float a, b;
-    swap_rows<false>(x, a, b);
-    swap_rows<true>(fmaxf(a, b), a, b);
-    return fmaxf(a, b);
 }
 
 // Per-lane DMA state.  A page is fetched as 16-byte chunks in two regions -- region A: the

@@ -113,6 +113,12 @@ def residual_pages(tail_lens) -> int:
     return RESIDUAL_FIXED_PAGES + (RESIDUAL_TAIL_PAGES * t + 63) // 127
 
 
+def scaled_pages(pages: int, page_elems: int) -> int:
+    """A cost of ``pages`` 128 x 128 pages in pages of ``page_elems`` (page_size x head_dim), at
+    least one (a cost of none stays none)."""
+    return max(1, round(pages * 128 * 128 / page_elems)) if pages > 0 else 0
+
+
 # Fixed cost of one split-K item, in packed pages: the workgroup's prologue (argument block, work
 # record, DMA set-up, q and tier table: the first page's barrier passes ≈8 us after the start on
 # c2 and c1, per-workgroup stamps), its epilogue (≈1.6 us) and its share of the cross-split reduce,
@@ -127,7 +133,8 @@ ALONE_FACTOR = 0.78
 
 
 @functools.lru_cache(maxsize=256)
-def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int) -> int:
+def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
+                     overhead: int = ITEM_OVERHEAD_PAGES) -> int:
     p = np.asarray(pages, dtype=np.int64)
     work = p + residual_pages
     top = max(1, -(-n_kv * int(work.sum()) // slots))
@@ -138,14 +145,15 @@ def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int) -
     wgs = n_kv * items.sum(axis=1)
     rounds = -(-wgs // slots)
     largest = (-(-work[None, :] // items)).max(axis=1)
-    cost = (rounds * (largest + ITEM_OVERHEAD_PAGES)).astype(np.float64)
+    cost = (rounds * (largest + overhead)).astype(np.float64)
     alone = wgs <= slots // 2
-    cost = np.where(alone, (largest + ITEM_OVERHEAD_PAGES) * ALONE_FACTOR, cost)
+    cost = np.where(alone, (largest + overhead) * ALONE_FACTOR, cost)
     cost = np.where((size[:, 0] > top) & ~alone, np.inf, cost)
     return int(size[int(np.argmin(cost)), 0])                          # ties: fewest items
 
 
-def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int, device=None) -> int:
+def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int, device=None,
+                           page_elems: int = 128 * 128) -> int:
     """Work per split-K item, in pages.  The decode kernel holds two workgroups per CU (the
     slots).  Items of ``total work / slots`` pages fill the slots once when every sequence's
     work (its pages plus its residual) divides evenly; with ragged lengths the per-sequence
@@ -153,12 +161,18 @@ def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int
     items.  The size is therefore the one, up to that one-round size, that minimises
     rounds x (largest item + the per-item cost), with ties going to fewer items -- or a larger
     size whose items leave every workgroup a CU of its own, when that costs less at
-    ``ALONE_FACTOR`` (small batches: c1 takes 5-page items instead of 3)."""
+    ``ALONE_FACTOR`` (small batches: c1 takes 5-page items instead of 3).
+
+    ``page_elems``: page_size x head_dim.  The per-item cost is the time of
+    ``ITEM_OVERHEAD_PAGES`` 128 x 128 pages, so smaller pages count more of themselves: 64-token
+    pages of head_dim 64 (8 sequences of 50 pages, 2 kv heads) take 4-page items, 15.0 us per
+    layer-step, instead of the 2-page ones of an unscaled cost, 18.2."""
     forced = env_int("LOGITFILL_AMD_PAGES_PER_SPLIT", 0)
     if forced > 0:
         return forced
     slots = 2 * (_cu_count(device) if device is not None else 256)
-    return _pages_per_split(tuple(int(x) for x in hist_pages), int(n_kv), int(residual_pages), slots)
+    return _pages_per_split(tuple(int(x) for x in hist_pages), int(n_kv), int(residual_pages), slots,
+                            scaled_pages(ITEM_OVERHEAD_PAGES, page_elems))
 
 
 # Of the two decode workgroups that share a CU, the one dispatched second runs this much slower
@@ -449,16 +463,21 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
     # q_len new tokens lengthen the residual (a chunk of 128 tokens more past a full page)
     res_pages = residual_pages(layer.tail_lens) + (max(layer.tail_lens, default=0) + q_len - 1) // P * (
         RESIDUAL_FIXED_PAGES + RESIDUAL_TAIL_PAGES)
+    page_elems = P * D
+    if page_elems != 128 * 128:
+        res_pages = scaled_pages(res_pages, page_elems)
     # workgroups per (item, kv head): one per tile of query rows
     tiles = -(-(manager.n_q // manager.n_kv * q_len) // MFMA_TILE_ROWS)
     if pages_per_split is None:
         # the split depends on the history, the residual cost, the environment's override and
-        # whether the matrix-core kernel's dispatch order applies: chosen again when one changes
-        age = kernel != _native.KERNEL_VALU and tiles == 1
+        # whether the dispatch order of decode_mfma.hip applies (its layout, one row tile): chosen
+        # again when one changes
+        age = (kernel != _native.KERNEL_VALU and tiles == 1
+               and P == layer.k_group_size == layer.v_group_size == D == 128)
         choice_key = (hist_pages, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"), age, tiles)
         cached = layer.__dict__.get("_lf_split_choice")
         if cached is None or cached[0] != choice_key:
-            size = choose_pages_per_split(list(hist_pages), layer.n_kv * tiles, res_pages, layer.device)
+            size = choose_pages_per_split(list(hist_pages), layer.n_kv * tiles, res_pages, layer.device, page_elems)
             if age and choice_key[2] is None:
                 cus = _cu_count(layer.device)
                 paired = paired_split(list(hist_pages), layer.n_kv, res_pages, cus, size)
