@@ -88,15 +88,6 @@ __device__ __forceinline__ int block_rank(int tier, int j, int q, int e) {
     return 32 * j + 4 * e + q;
 }
 
-// A choice among values.  The values are function arguments, so they are there before the choice:
-// written as ?: over kernel arguments or captured variables, the compiler turns it into a choice of
-// addresses and one load -- of the argument block from scratch, and the wait for that load is a wait
-// for every DMA issued before it.
-template <class T>
-__device__ __forceinline__ T pick3(bool one, bool two, T a, T b, T c) { return two ? c : one ? b : a; }
-template <class T>
-__device__ __forceinline__ T pick4(bool one, bool two, bool three, T a, T b, T c, T d) { return three ? d : two ? c : one ? b : a; }
-
 // (tier, rank) of position pos of the K dimension; k1, k2, k3: the first K-steps of tiers 1 to 3.
 __device__ __forceinline__ void pos_slot(int k1, int k2, int k3, int pos, int& tier, int& rank) {
     const int step = pos >> 5;
@@ -119,14 +110,6 @@ __device__ __forceinline__ uint32_t in_vgpr(uint32_t x) {
     asm volatile("" : "+v"(x));
     return x;
 }
-// A wave-uniform value as a value in SGPRs (not a load that could be repeated or redirected).
-__device__ __forceinline__ int in_sgpr(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ const unsigned char* in_sgpr(const unsigned char* x) {
-    const uint64_t u = reinterpret_cast<uint64_t>(x);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(u)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(u >> 32));
-    return reinterpret_cast<const unsigned char*>(static_cast<uint64_t>(hi) << 32 | lo);
-}
-
 // x again, opaque to the compiler: what is derived from it is computed where it is used instead of
 // being hoisted out of the token loop into registers (and spilled).
 __device__ __forceinline__ int fresh(int x) {

@@ -77,6 +77,26 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// ---- values a lane chooses among ----------------------------------------------------
+
+// A wave-uniform value as a value in SGPRs (not a load that could be repeated or redirected).
+__device__ __forceinline__ int in_sgpr(int x) { return __builtin_amdgcn_readfirstlane(x); }
+template <class T>
+__device__ __forceinline__ T* in_sgpr(T* x) {
+    const uint64_t u = reinterpret_cast<uint64_t>(x);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(u)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(u >> 32));
+    return reinterpret_cast<T*>(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
+// A choice among values.  The values are function arguments, so they are there before the choice:
+// written as ?: over kernel arguments or captured variables, the compiler turns it into a choice of
+// addresses and one load -- of the argument block from scratch, and the wait for that load is a wait
+// for every DMA issued before it.
+template <class T>
+__device__ __forceinline__ T pick3(bool one, bool two, T a, T b, T c) { return two ? c : one ? b : a; }
+template <class T>
+__device__ __forceinline__ T pick4(bool one, bool two, bool three, T a, T b, T c, T d) { return three ? d : two ? c : one ? b : a; }
+
 // ---- layout offsets (reference byte layout, capacity strided) -----------
 
 // Row (b, h, token) of a [batch][n_kv][cap_tokens][...] array.
