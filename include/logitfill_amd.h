@@ -307,6 +307,18 @@ int32_t lf_append_token(void* tail_k, void* tail_v, int32_t tail_dtype, int32_t 
                         int32_t head_dim, void* stream);
 
 /*
+ * Rows of new tokens into the residual pages (the copies of a commit of several tokens, reference
+ * src/logitfill/packed/cache.py:48-62).  ``segs`` (HOST, n_segs x 4, read during the call) lists
+ * (sequence b, first source token, first page row, tokens): for every kv head those rows of k_src /
+ * v_src, whose element strides per sequence, head and token are k_strides / v_strides [3] (unit
+ * channel stride), go to tail_k / tail_v [batch][n_kv][tail_cap][head_dim] of the same ``dtype``.
+ * ``every`` 1: the one segment of ``segs`` for every sequence of the batch (its b is ignored).
+ */
+int32_t lf_fill_tail(void* tail_k, void* tail_v, const void* k_src, const void* v_src, int32_t dtype,
+                     const int64_t* k_strides, const int64_t* v_strides, int32_t tail_cap, const int32_t* segs,
+                     int32_t n_segs, int32_t every, int32_t batch, int32_t n_kv, int32_t head_dim, void* stream);
+
+/*
  * Layout helpers on the device (building blocks of the page packers, for callers of the
  * reference's layout module).  All arrays are contiguous device memory.
  *

@@ -114,6 +114,8 @@ _SIGNATURES = {
     "lf_decode_attention_noalloc": (c_int32, [POINTER(PackedLayer), POINTER(DecodeArgs), c_void_p]),
     "lf_append_token": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int32,
                                   c_int32, c_int32, c_int32, c_void_p]),
+    "lf_fill_tail": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_int32, c_void_p,
+                               c_int32, c_int32, c_int32, c_int32, c_int32, c_void_p]),
     "lf_noalloc_scratch_bytes": (c_int64, []),
 }
 

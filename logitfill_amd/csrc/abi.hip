@@ -28,6 +28,9 @@ int launch_unpack_ints(const int32_t* words, int64_t rows, int n_words, int coun
 int launch_append_token(void* tail_k, void* tail_v, int tail_dtype, int tail_cap, int32_t* tail_len,
                         const void* k_new, const void* v_new, int new_dtype, int batch, int n_kv, int head_dim,
                         hipStream_t stream);
+int launch_fill_tail(void* tail_k, void* tail_v, const void* k_src, const void* v_src, int dtype,
+                     const int64_t* k_strides, const int64_t* v_strides, int tail_cap, const int32_t* segs, int n_segs,
+                     int every, int n_kv, int head_dim, hipStream_t stream);
 }  // namespace lf
 
 namespace {
@@ -268,6 +271,22 @@ int32_t lf_append_token(void* tail_k, void* tail_v, int32_t tail_dtype, int32_t 
     if (!tail_k || !tail_v || !tail_len || !k_new || !v_new) return LF_E_NULL;
     return lf::launch_append_token(tail_k, tail_v, tail_dtype, tail_cap, tail_len, k_new, v_new, new_dtype, batch,
                                    n_kv, head_dim, static_cast<hipStream_t>(stream));
+}
+
+int32_t lf_fill_tail(void* tail_k, void* tail_v, const void* k_src, const void* v_src, int32_t dtype,
+                     const int64_t* k_strides, const int64_t* v_strides, int32_t tail_cap, const int32_t* segs,
+                     int32_t n_segs, int32_t every, int32_t batch, int32_t n_kv, int32_t head_dim, void* stream) {
+    if (!valid_dtype(dtype)) return LF_E_DTYPE;
+    if (batch <= 0 || n_kv <= 0 || n_kv > 65535 || head_dim <= 0 || tail_cap <= 0 || n_segs < 0) return LF_E_SHAPE;
+    if (every != 0 && (every != 1 || n_segs != 1)) return LF_E_SHAPE;
+    if (n_segs == 0) return LF_OK;
+    if (!tail_k || !tail_v || !k_src || !v_src || !k_strides || !v_strides || !segs) return LF_E_NULL;
+    for (int32_t i = 0; i < n_segs; ++i) {
+        const int32_t* s = segs + 4 * i;
+        if (s[0] < 0 || s[0] >= batch || s[1] < 0 || s[2] < 0 || s[3] < 0 || s[2] > tail_cap - s[3]) return LF_E_SHAPE;
+    }
+    return lf::launch_fill_tail(tail_k, tail_v, k_src, v_src, dtype, k_strides, v_strides, tail_cap, segs, n_segs,
+                                every ? batch : 0, n_kv, head_dim, static_cast<hipStream_t>(stream));
 }
 
 int32_t lf_asymmetric_codes(const void* x, int32_t dtype, int64_t n_groups, int32_t group, int32_t bits,

@@ -19,9 +19,11 @@ batch != 1, ``cache.py:136-137``); ``commit`` then takes ``[batch, n_kv, T, D]``
 """
 from __future__ import annotations
 
+import ctypes
 import os
 from typing import Optional
 
+import numpy as np
 import torch
 
 from logitfill_amd import _native
@@ -223,7 +225,14 @@ class _LayerStore:
         """int32 ``[B]`` residual lengths on the device, re-uploaded (asynchronously, from pinned
         memory, on the current stream) after they change."""
         if self._tail_dirty or self._tail_len_dev is None:
-            self._tail_len_dev = _native.upload(self.tail_lens, torch.int32, self.device)
+            if min(self.tail_lens) == max(self.tail_lens):
+                # one value: a fill in place of the staging and copy, into the tensor that is there
+                # (the decode's argument block keeps its address)
+                if self._tail_len_dev is None:
+                    self._tail_len_dev = torch.empty(self.batch, dtype=torch.int32, device=self.device)
+                self._tail_len_dev.fill_(self.tail_lens[0])
+            else:
+                self._tail_len_dev = _native.upload(self.tail_lens, torch.int32, self.device)
             self._tail_dirty = False
         return self._tail_len_dev
 
@@ -283,66 +292,97 @@ class _LayerStore:
             key = key.to(self._tail_k.dtype)
         if value.dtype != self._tail_v.dtype:
             value = value.to(self._tail_v.dtype)
-        key = key.detach()
-        value = value.detach()
+        key = self._rows_here(key)
+        value = self._rows_here(value)
 
-        tail_jobs, src_jobs, rest = [], [], {}
-        fill: dict[tuple[int, int], list[int]] = {}
-        hist_pages = [h // P for h in self.hist_lens]
-        new_tail = list(self.tail_lens)
-        for b in range(B):
-            Tb = lens[b]
-            if Tb == 0:
+        # Where every sequence's tokens go: rows of residual pages (b, source token, page row, tokens),
+        # written before or after the packing, and pages to pack (b, source token, destination page),
+        # from the residual page it completes or straight from the source.
+        tails = self.tail_lens
+        hist = [h // P for h in self.hist_lens]
+        same = lengths is None and min(tails) == max(tails)  # one plan for every sequence
+        seqs = [0] if same else [b for b in range(B) if lens[b]]
+        over = {b: lens[b] - (P - tails[b]) for b in seqs}   # tokens past the end of the residual page
+        # a deferring store on a step that only completes residual pages leaves them full in the
+        # residual buffers until flush()
+        defer = self.defer_flush and max(over.values()) == 0
+        before, after, plan = [], [], {}
+        new_tail = list(tails)
+        for b in seqs:
+            tl, start = tails[b], 0
+            if over[b] < 0 or defer and over[b] == 0:
+                before.append((b, 0, tl, lens[b]))
+                new_tail[b] = tl + lens[b]
                 continue
-            tl = self.tail_lens[b]
-            n1 = min(Tb, P - tl)
-            fill.setdefault((tl, n1), []).append(b)
-            pos = n1
-            if tl + n1 == P:
-                tail_jobs.append((b, 0, hist_pages[b]))
-                hist_pages[b] += 1
-                new_tail[b] = 0
-            else:
-                new_tail[b] = tl + n1
-            while Tb - pos >= P:
-                src_jobs.append((b, pos, hist_pages[b]))
-                hist_pages[b] += 1
-                pos += P
-            if pos < Tb:
-                rest[b] = (pos, Tb)
-                new_tail[b] = Tb - pos
-        # 1) complete the residual pages
-        for (tl, n1), bs in fill.items():
-            if len(bs) == B:
-                self._tail_k[:, :, tl:tl + n1].copy_(key[:, :, :n1])
-                self._tail_v[:, :, tl:tl + n1].copy_(value[:, :, :n1])
-            else:
-                idx = _native.upload(bs, torch.int64, self.device)
-                self._tail_k[idx, :, tl:tl + n1] = key[idx, :, :n1]
-                self._tail_v[idx, :, tl:tl + n1] = value[idx, :, :n1]
-        # 2) pack full pages in place -- or, for a deferring store on a step that only completes
-        # residual pages, leave them full in the residual buffers until flush()
-        defer = self.defer_flush and bool(tail_jobs) and not src_jobs and not rest
-        if tail_jobs or src_jobs:
-            self.reserve(max(hist_pages) * P)
-            if defer:
-                for b, _, page in tail_jobs:
-                    self._pending.append((b, page))
-                    hist_pages[b] -= 1
-                    new_tail[b] = P
-            else:
-                if tail_jobs:
-                    self._pack(self._tail_k, self._tail_v, tail_jobs)
-                if src_jobs:
-                    self._pack(key, value, src_jobs)
-        # 3) start the next residual pages
-        for b, (pos, end) in rest.items():
-            n = end - pos
-            self._tail_k[b, :, :n].copy_(key[b, :, pos:end])
-            self._tail_v[b, :, :n].copy_(value[b, :, pos:end])
-        self.hist_lens = [p * P for p in hist_pages]
+            if tl:
+                start = P - tl
+                before.append((b, 0, tl, start))
+            pages, rest = divmod(lens[b] - start, P)
+            if rest:  # (a page packed from the residual buffer is read before these rows replace it)
+                (after if tl else before).append((b, start + pages * P, 0, rest))
+            plan[b] = (start, pages)
+            new_tail[b] = rest
+        if same:
+            new_tail = [new_tail[0]] * B
+            if plan:
+                plan = {b: plan[0] for b in range(B)}
+            elif new_tail[0] < P:  # rows of residual pages only
+                self._fill_tail(key, value, before, True)
+                self.tail_lens = new_tail
+                self._tail_dirty = True
+                return
+        tail_jobs, src_jobs = [], None
+        if plan:
+            tail_jobs = [(b, 0, hist[b]) for b, (start, _) in plan.items() if start]
+            seq, start, pages = (np.array(x, dtype=np.int32) for x in
+                                 (list(plan), [x for x, _ in plan.values()], [n for _, n in plan.values()]))
+            first = np.array([hist[b] for b in plan], dtype=np.int32) + (start > 0)  # the source's first page
+            if pages.any():
+                at = np.arange(pages.sum(), dtype=np.int32) - np.repeat(np.cumsum(pages) - pages, pages)
+                src_jobs = np.stack([np.repeat(seq, pages), np.repeat(start, pages) + P * at,
+                                     np.repeat(first, pages) + at], 1).astype(np.int32)
+            for b, h in zip(plan, (first + pages).tolist()):
+                hist[b] = h
+        done = [b for b in range(B) if new_tail[b] == P]  # full, deferred
+        self._fill_tail(key, value, before, same)
+        if plan or done:
+            self.reserve(max([hist[b] for b in plan] + [hist[b] + 1 for b in done]) * P)
+        self._pending.extend((b, hist[b]) for b in done)
+        if tail_jobs:
+            self._pack(self._tail_k, self._tail_v, tail_jobs)
+        if src_jobs is not None:
+            self._pack(key, value, src_jobs)
+        self._fill_tail(key, value, after, same)
+        self.hist_lens = [p * P for p in hist]
         self.tail_lens = new_tail
         self._tail_dirty = True
+
+    def _rows_here(self, t: torch.Tensor) -> torch.Tensor:
+        """``t`` as the kernels read it: on this device, unit channel stride, no autograd."""
+        t = t.detach()
+        if t.device != self.device:
+            t = t.to(self.device)
+        return t if t.stride(-1) == 1 else t.contiguous()
+
+    def _fill_tail(self, key: torch.Tensor, value: torch.Tensor, rows: list, same: bool) -> None:
+        """Copy ``rows`` (b, source token, page row, tokens) into the residual pages, all of them in
+        one launch; ``same``: the one entry holds for every sequence."""
+        if not rows:
+            return
+        tk, tv = self._tail_k, self._tail_v
+        if tk.dtype != tv.dtype or tk.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+            for b, tok, row, n in rows:  # (outside the kernels' types: copies)
+                at = slice(None) if same else slice(b, b + 1)
+                tk[at, :, row:row + n].copy_(key[at, :, tok:tok + n])
+                tv[at, :, row:row + n].copy_(value[at, :, tok:tok + n])
+            return
+        segs = (ctypes.c_int32 * (4 * len(rows)))(*[x for row in rows for x in row])
+        ks, vs = (ctypes.c_int64 * 3)(*key.stride()[:3]), (ctypes.c_int64 * 3)(*value.stride()[:3])
+        st = _native.load().lf_fill_tail(
+            tk.data_ptr(), tv.data_ptr(), key.data_ptr(), value.data_ptr(), _native.dtype_code(tk.dtype), ks, vs,
+            self.page_size, segs, len(rows), 1 if same else 0, self.batch, self.n_kv, self.head_dim,
+            _native.current_stream_ptr(self.device))
+        _native.check(st, "lf_fill_tail")
 
     def _append_one(self, key: torch.Tensor, value: torch.Tensor) -> None:
         """One token per sequence into residual pages that stay below full: ``lf_append_token``
@@ -379,20 +419,25 @@ class _LayerStore:
 
     def _complete_pending(self) -> None:
         P = self.page_size
-        for b, _ in self._pending:
-            self.hist_lens[b] += P
-            self.tail_lens[b] = 0
+        if len(self._pending) == self.batch:  # every sequence's page
+            self.hist_lens = [h + P for h in self.hist_lens]
+            self.tail_lens = [0] * self.batch
+        else:
+            for b, _ in self._pending:
+                self.hist_lens[b] += P
+                self.tail_lens[b] = 0
         self._pending = []
         self._tail_dirty = True
 
-    def _pack(self, k_src: torch.Tensor, v_src: torch.Tensor, jobs: list) -> None:
+    def _pack(self, k_src: torch.Tensor, v_src: torch.Tensor, jobs) -> None:
+        """Pack the pages of ``jobs`` (b, source token, destination page), a list or an [n, 3] array."""
         if k_src.stride(-1) != 1:
             k_src = k_src.contiguous()
         if v_src.stride(-1) != 1:
             v_src = v_src.contiguous()
         if k_src.stride() != v_src.stride():
             k_src, v_src = k_src.contiguous(), v_src.contiguous()
-        jobs_dev = _native.upload([v for job in jobs for v in job], torch.int32, self.device)
+        jobs_dev = _native.upload(np.asarray(jobs, dtype=np.int32).reshape(-1), torch.int32, self.device)
         st = _native.load().lf_pack_pages(
             self.layer_struct(), k_src.data_ptr(), v_src.data_ptr(), _native.dtype_code(k_src.dtype),
             k_src.stride(0), k_src.stride(1), k_src.stride(2), jobs_dev.data_ptr(), len(jobs),
@@ -520,8 +565,15 @@ class PackedKVManager:
         if st is None:
             dev_structs = _native.upload(bytes(structs), torch.uint8, self.device)
             dev_srcs = _native.upload(bytes(srcs), torch.uint8, self.device)
-            jobs = [(i, b, 0, page) for i, layer in enumerate(todo) for b, page in layer._pending]
-            jobs_dev = _native.upload([v for job in jobs for v in job], torch.int32, self.device)
+            # (layer, b, source token 0, page) of every pending page; as a rule the layers' are the same
+            parts = [np.array(layer._pending, dtype=np.int32) for layer in todo[:1]]
+            for i in range(1, n):
+                alike = todo[i]._pending == todo[i - 1]._pending
+                parts.append(parts[-1] if alike else np.array(todo[i]._pending, dtype=np.int32))
+            jobs = np.zeros((sum(map(len, parts)), 4), dtype=np.int32)
+            jobs[:, 0] = np.repeat(np.arange(n, dtype=np.int32), [len(p) for p in parts])
+            jobs[:, 1::2] = np.concatenate(parts)
+            jobs_dev = _native.upload(jobs.reshape(-1), torch.int32, self.device)
             st = _native.load().lf_pack_pages_multi(
                 dev_structs.data_ptr(), structs, dev_srcs.data_ptr(), srcs, n, _native.dtype_code(dtypes.pop()),
                 jobs_dev.data_ptr(), len(jobs), _native.current_stream_ptr(self.device))
