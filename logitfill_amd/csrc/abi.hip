@@ -13,6 +13,7 @@ int launch_pack_pages_multi(const lf_packed_layer* layers_dev, const lf_packed_l
                             int src_dtype, const int32_t* jobs, int n_jobs, hipStream_t stream);
 int launch_decode_valu(const DecodeParams& p, hipStream_t stream);
 int launch_decode_mfma(const DecodeParams& p, hipStream_t stream, bool* handled);
+int launch_decode_rows(const DecodeParams& p, hipStream_t stream, bool* handled);
 int launch_decode_tiled(const DecodeParams& p, hipStream_t stream, bool* handled);
 int launch_dequantize(const lf_packed_layer& L, int b, int tokens, float* k_out, float* v_out,
                       hipStream_t stream);
@@ -125,6 +126,8 @@ int32_t decode_checked(const lf_packed_layer* layer, const lf_decode_args* args,
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (A.kernel != 1) {
         bool handled = false;
+        const int rr = A.kernel == 0 ? launch_decode_rows(p, s, &handled) : LF_OK;
+        if (handled) return rr;
         const int r = launch_decode_mfma(p, s, &handled);
         if (handled || A.kernel == 2) return handled ? r : LF_E_UNSUPPORTED;
         const int rt = launch_decode_tiled(p, s, &handled);

@@ -199,6 +199,16 @@ __device__ __forceinline__ void commit_new_rows(const DecodeParams& p, int b, in
     }
 }
 
+// Where many query rows per kv head go to decode_rows.hip instead of decode_mfma.hip's tiles of 8:
+// from 6 tiles up and 3 000 page-tiles (pages x kv heads x tiles of 8 rows) in the call.  Below, the
+// one workgroup per CU of decode_rows.hip pays its longer start on too few pages, or its 64-row tile
+// is mostly empty (us per layer-step, decode_mfma / decode_rows, 28 q on 4 kv heads unless stated):
+// 28 rows x 125 pages 22.5 / 26.3, x 770 pages 74.1 / 73.4; 35 rows x 770 85.1 / 86.2; 56 rows x 125
+// (3 500) 38.2 / 30.6, x 770 110 / 91; 224 x 125 88 / 47; 64 rows, 2 kv heads, 124 pages (1 984) 23.1 /
+// 26.6; 120 rows, 2 kv heads, 28 pages (840) 19.2 / 21.4.
+constexpr int kRowsTiles = 6;
+constexpr int kRowsWork = 3000;
+
 // Merge the partials of every sequence into ``out`` (enqueued after a decode kernel).  With the
 // host copy of seq_work and at most LF_INLINE_SEQ sequences, the (first, count) pairs go into
 // the reduce kernel's arguments.

@@ -134,7 +134,7 @@ ALONE_FACTOR = 0.78
 
 @functools.lru_cache(maxsize=256)
 def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
-                     overhead: int = ITEM_OVERHEAD_PAGES) -> int:
+                     overhead: int = ITEM_OVERHEAD_PAGES, per_cu: int = 2) -> int:
     p = np.asarray(pages, dtype=np.int64)
     work = p + residual_pages
     top = max(1, -(-n_kv * int(work.sum()) // slots))
@@ -146,14 +146,15 @@ def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
     rounds = -(-wgs // slots)
     largest = (-(-work[None, :] // items)).max(axis=1)
     cost = (rounds * (largest + overhead)).astype(np.float64)
-    alone = wgs <= slots // 2
+    alone = wgs <= (slots // 2 if per_cu == 2 else 0)
     cost = np.where(alone, (largest + overhead) * ALONE_FACTOR, cost)
-    cost = np.where((size[:, 0] > top) & ~alone, np.inf, cost)
+    if per_cu == 2:
+        cost = np.where((size[:, 0] > top) & ~alone, np.inf, cost)
     return int(size[int(np.argmin(cost)), 0])                          # ties: fewest items
 
 
 def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int, device=None,
-                           page_elems: int = 128 * 128) -> int:
+                           page_elems: int = 128 * 128, per_cu: int = 2) -> int:
     """Work per split-K item, in pages.  The decode kernel holds two workgroups per CU (the
     slots).  Items of ``total work / slots`` pages fill the slots once when every sequence's
     work (its pages plus its residual) divides evenly; with ragged lengths the per-sequence
@@ -166,13 +167,14 @@ def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int
     ``page_elems``: page_size x head_dim.  The per-item cost is the time of
     ``ITEM_OVERHEAD_PAGES`` 128 x 128 pages, so smaller pages count more of themselves: 64-token
     pages of head_dim 64 (8 sequences of 50 pages, 2 kv heads) take 4-page items, 15.0 us per
-    layer-step, instead of the 2-page ones of an unscaled cost, 18.2."""
+    layer-step, instead of the 2-page ones of an unscaled cost, 18.2.  ``per_cu``: workgroups a
+    CU holds (one of decode_rows.hip)."""
     forced = env_int("LOGITFILL_AMD_PAGES_PER_SPLIT", 0)
     if forced > 0:
         return forced
-    slots = 2 * (_cu_count(device) if device is not None else 256)
+    slots = per_cu * (_cu_count(device) if device is not None else 256)
     return _pages_per_split(tuple(int(x) for x in hist_pages), int(n_kv), int(residual_pages), slots,
-                            scaled_pages(ITEM_OVERHEAD_PAGES, page_elems))
+                            scaled_pages(ITEM_OVERHEAD_PAGES, page_elems), per_cu)
 
 
 # Of the two decode workgroups that share a CU, the one dispatched second runs this much slower
@@ -467,17 +469,26 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
     if page_elems != 128 * 128:
         res_pages = scaled_pages(res_pages, page_elems)
     # workgroups per (item, kv head): one per tile of query rows
-    tiles = -(-(manager.n_q // manager.n_kv * q_len) // MFMA_TILE_ROWS)
+    rows = manager.n_q // manager.n_kv * q_len
+    default_layout = P == layer.k_group_size == layer.v_group_size == D == 128
+    tiles = -(-rows // MFMA_TILE_ROWS)
+    # decode_rows.hip takes the call
+    wide = (tiles >= ROWS_TILES and sum(hist_pages) * layer.n_kv * tiles >= ROWS_WORK and default_layout
+            and kernel == _native.KERNEL_AUTO and query.dtype != torch.float32)
+    if wide:
+        tiles = -(-rows // rows_tile(rows))
+        # a dense chunk of 128 tail and new tokens costs about a page there
+        res_pages = 1 + -(-(max(layer.tail_lens, default=0) + q_len) // P)
     if pages_per_split is None:
         # the split depends on the history, the residual cost, the environment's override and
         # whether the dispatch order of decode_mfma.hip applies (its layout, one row tile): chosen
         # again when one changes
-        age = (kernel != _native.KERNEL_VALU and tiles == 1
-               and P == layer.k_group_size == layer.v_group_size == D == 128)
-        choice_key = (hist_pages, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"), age, tiles)
+        age = kernel != _native.KERNEL_VALU and tiles == 1 and not wide and default_layout
+        choice_key = (hist_pages, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"), age, tiles, wide)
         cached = layer.__dict__.get("_lf_split_choice")
         if cached is None or cached[0] != choice_key:
-            size = choose_pages_per_split(list(hist_pages), layer.n_kv * tiles, res_pages, layer.device, page_elems)
+            size = choose_pages_per_split(list(hist_pages), layer.n_kv * tiles, res_pages, layer.device, page_elems,
+                                          1 if wide else 2)
             if age and choice_key[2] is None:
                 cus = _cu_count(layer.device)
                 paired = paired_split(list(hist_pages), layer.n_kv, res_pages, cus, size)
@@ -587,6 +598,16 @@ def _kernel_attention(manager, layer_idx: int, query: torch.Tensor, key_new: tor
 # Query rows per workgroup of the matrix-core decode kernel: rows beyond it ((n_q / n_kv) * q_len
 # per kv head) run as further row tiles, each a workgroup of its own over the same pages.
 MFMA_TILE_ROWS = 8
+
+# Calls of at least this many tiles of MFMA_TILE_ROWS rows and this many page-tiles (pages x kv heads
+# x tiles) run decode_rows.hip (kRowsTiles, kRowsWork there, with the measurements).
+ROWS_TILES = 6
+ROWS_WORK = 3000
+
+
+def rows_tile(rows: int) -> int:
+    """Query rows per workgroup of decode_rows.hip for ``rows`` rows per kv head."""
+    return 128 if rows > 64 else 64
 
 
 def valu_tile_rows(head_dim: int) -> int:

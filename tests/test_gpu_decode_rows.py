@@ -1,0 +1,52 @@
+"""Decode with many query rows per kv head (decode_rows.hip) against float64 attention over the
+device's own history, at the edges of its row tiles, K-steps and residual chunks."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from logitfill_amd import _native
+from logitfill_amd.packed.reference import decode_into
+from tests.test_gpu_tiled import _decode, _float64, _rel, _setup
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n_q,n_kv,lengths,q_len,dtype,tb,pps", [
+    (14, 2, [250 * 128 + 40, 128, 60], 9, torch.bfloat16, 3.0, None),    # 63 rows: 64-row tile; no page
+    (41, 1, [510 * 128 + 127], 1, torch.float16, 4.0, 100),              # the fewest rows, one token
+    (64, 2, [140 * 128, 70 * 128 + 1], 2, torch.bfloat16, 2.5, None),    # exactly 64
+    (40, 8, [45 * 128 + 127, 128], 13, torch.float16, 2.5, None),        # 65 rows: 128-row tile
+    (28, 4, [6 * 128 + 17, 3 * 128], 130, torch.bfloat16, 3.0, None),    # 910 rows, residual of two chunks
+    (8, 8, [12 * 128, 50], 300, torch.float16, 2.5, 1),                  # no GQA, three chunks, no tail / tail
+    (64, 1, [520 * 128], 1, torch.bfloat16, 2.5, 520),                   # one long item
+])
+def test_many_rows(gpu, n_q, n_kv, lengths, q_len, dtype, tb, pps):
+    """float32 output within 2e-5 of float64 in the 2-norm: fp16 hi + lo operands keep 22 bits
+    (2.4e-7 a term) and the largest scores here are about 30."""
+    mgr, _, _, q, kn, vn = _setup(gpu, 128, 128, 128, 128, n_q, n_kv, lengths, q_len, dtype, tb)
+    want = _float64(mgr, q, kn, vn)
+    rel = _rel(_decode(mgr, q, kn, vn, _native.KERNEL_AUTO, pps), want)
+    print(f"rel {rel:.2e}")
+    assert rel < 2e-5
+
+
+@pytest.mark.parametrize("level", [0, 1, 2])
+def test_many_rows_single_tier(gpu, level):
+    """Every channel in one tier (int8: 32 words a token, 8 K-steps)."""
+    mgr, _, _, q, kn, vn = _setup(gpu, 128, 128, 128, 128, 72, 1, [340 * 128 + 3], 1, torch.bfloat16,
+                                  levels=np.full((1, 128), level))
+    assert _rel(_decode(mgr, q, kn, vn, _native.KERNEL_AUTO), _float64(mgr, q, kn, vn)) < 2e-5
+
+
+def test_many_rows_commit(gpu):
+    """The folded commit: the new rows land in the tail and the device length advances."""
+    mgr, _, _, q, kn, vn = _setup(gpu, 128, 128, 128, 128, 28, 4, [80 * 128 + 17], 12, torch.bfloat16)
+    layer = mgr.layers[0]
+    out = torch.empty_like(q)
+    assert decode_into(mgr, 0, q, kn, vn, 128 ** -0.5, out, commit=True)
+    torch.cuda.synchronize()
+    tk, tv = layer.tail_buffers()
+    assert layer.tail_lens == [29] and layer.tail_len_device().tolist() == [29]
+    assert torch.equal(tk[:, :, 17:29], kn) and torch.equal(tv[:, :, 17:29], vn)
