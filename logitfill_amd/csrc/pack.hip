@@ -869,6 +869,299 @@ int launch_fast_multi(const PackMultiArgs& m, bool half, dim3 grid, size_t lds, 
                                       lds, m, stream);
 }
 
+// ---------------------------------------------------------------------------------------
+// Tiled path for the other layouts of 2-byte inputs with 16-byte aligned rows: head_dim 64, 128 or
+// 256, Key groups of 32 to 128 tokens in whole 32-token pieces, Value groups of whole 32-channel
+// pieces (any Value width).  One workgroup of 256 threads per block of ``tb`` tokens (one or more
+// whole Key groups) of a page, kv head and kind (Key or Value); the element arithmetic is the fast
+// path's.  Key: the block is staged in LDS, a thread holds U pieces of (channel, 32 tokens) in
+// registers, the pieces' minima and maxima meet in LDS, and the codes go out as bytes over the
+// staged block, from which the words are assembled.  Value: a thread holds (token, 32 channels),
+// straight from memory; a group's pieces are neighbouring lanes.
+// Bound: memory, as the fast path.  The general kernel behind it divides per element, reads each
+// element from LDS twice and takes Key and Value one after the other: 2 184 pages of 64 tokens x 128
+// channels (Key groups of 32, int4 Values; 71 MB read, 40 MB written) 76 us, this one 34 (3.3 TB/s).
+// ---------------------------------------------------------------------------------------
+struct TileLds {
+    int ldc, pmm, cpos, tidx, total;  // code row bytes; offsets
+};
+
+__device__ __host__ inline TileLds tile_lds(const lf_packed_layer& L, int tb) {
+    TileLds t;
+    t.ldc = code_segs(L).seg[3] + 16;
+    const int codes = tb * t.ldc, page = tb * L.head_dim * 2;
+    t.pmm = ((codes > page ? codes : page) + 15) & ~15;
+    t.cpos = t.pmm + (tb / 32) * L.head_dim * 8;
+    t.tidx = t.cpos + L.head_dim * 2;
+    t.total = t.tidx + ((L.k_width[3] * 2 + 15) & ~15) + 16;
+    return t;
+}
+
+constexpr int kTileThreads = 256;
+
+// i / w = i * r >> 20 for i < 128 w, w < 90 (r = ceil(2^20 / w)).
+__device__ __forceinline__ uint32_t tile_rcp(int w) { return ((1u << 20) + w - 1) / w; }
+
+template <int Bits>
+__device__ __forceinline__ void tile_words(const uint8_t* codes, int ldc, int seg, int kw, int cnt, int tb, int32_t* out) {
+    if (kw == 0) return;
+    constexpr int kPer = 32 / Bits;
+    const uint32_t r = __builtin_amdgcn_readfirstlane(tile_rcp(kw));
+    for (int i = threadIdx.x; i < tb * kw; i += kTileThreads) {
+        const int tok = static_cast<int>(i * r >> 20), w = i - tok * kw;
+        const int nv = min(max(cnt - kPer * w, 0), kPer);
+        const uint32_t keep = nv >= kPer ? 0xffffffffu : (1u << (Bits * nv)) - 1u;
+        const uint8_t* src = codes + tok * ldc + seg + kPer * w;
+        uint32_t word;
+        if constexpr (Bits == 2) word = word_int2(*reinterpret_cast<const uint4*>(src));
+        else if constexpr (Bits == 4) word = word_int4(*reinterpret_cast<const uint2*>(src));
+        else word = *reinterpret_cast<const uint32_t*>(src);
+        out[i] = static_cast<int32_t>(word & keep);
+    }
+}
+
+// 32 channels of a token, Bits per code, into out (Bits words).
+template <int Bits>
+__device__ __forceinline__ void tile_value_words(const float (&v)[32], float lo, float sc, float y, bool magic, int32_t* out) {
+    constexpr int kPer = 32 / Bits;
+    constexpr float kQmax = static_cast<float>((1 << Bits) - 1);
+    uint32_t w[Bits];
+#pragma unroll
+    for (int j = 0; j < Bits; ++j) {
+        w[j] = 0;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const float x = v[kPer * j + i];
+            const uint32_t code = magic ? magic_code(x, lo, sc, y) & 0xffu : fast_code(x, lo, sc, y, kQmax);
+            w[j] |= code << (Bits * i);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < Bits; j += 2) reinterpret_cast<uint2*>(out)[j / 2] = make_uint2(w[j], w[j + 1]);
+}
+
+struct PackTileArgs {
+    PackJobArgs a;
+    int tb;  // tokens of a block
+};
+
+template <bool IsHalf, int U>
+__global__ __launch_bounds__(kTileThreads) void pack_tile_kernel(PackTileArgs ta) {
+    const PackJobArgs& a = ta.a;
+    const lf_packed_layer& L = a.L;
+    const int job = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, tb = ta.tb;
+    const bool value = (blockIdx.z & 1) != 0;
+    const int t0 = static_cast<int>(blockIdx.z >> 1) * tb;  // the block's first token of the page
+    const int b = a.jobs[3 * job], page = a.jobs[3 * job + 2];
+    const int64_t tok0 = a.jobs[3 * job + 1] + t0;
+    const int D = L.head_dim;
+    const int64_t row0 = tok_row(L, b, h, static_cast<int64_t>(page) * L.page_size + t0);
+    const int64_t off = b * a.sb + h * a.sh + tok0 * a.st;
+    extern __shared__ __align__(16) unsigned char smem[];
+
+    if (value) {
+        const uint16_t* src = static_cast<const uint16_t*>(a.v_src) + off;
+        const int parts = D / 32;
+        for (int u0 = 0; u0 < tb * parts; u0 += kTileThreads) {
+            const int u = u0 + tid;
+            const bool live = u < tb * parts;
+            const int tok = live ? u / parts : 0, part = u & (parts - 1);
+            uint4 r[4];
+            const uint4* p = reinterpret_cast<const uint4*>(src + tok * a.st + 32 * part);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[i] = p[i];
+            float v[32];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                pair_f32<IsHalf>(r[i].x, v[8 * i + 0], v[8 * i + 1]);
+                pair_f32<IsHalf>(r[i].y, v[8 * i + 2], v[8 * i + 3]);
+                pair_f32<IsHalf>(r[i].z, v[8 * i + 4], v[8 * i + 5]);
+                pair_f32<IsHalf>(r[i].w, v[8 * i + 6], v[8 * i + 7]);
+            }
+            if (L.bit_v >= 16) {
+                if (!live) continue;
+                uint16_t* out = L.v_value16 + (row0 + tok) * D + 32 * part;
+#pragma unroll
+                for (int i = 0; i < 32; i += 2)
+                    *reinterpret_cast<uint32_t*>(out + i) = f32_to_f16(v[i]) | static_cast<uint32_t>(f32_to_f16(v[i + 1])) << 16;
+                continue;
+            }
+            float lo, hi;
+            minmax32(v, lo, hi);
+            const int group = L.v_group / 32;  // pieces of a group: neighbouring lanes
+            for (int m = 1; m < group; m <<= 1) {
+                lo = fminf(lo, __shfl_xor(lo, m, kWave));
+                hi = fmaxf(hi, __shfl_xor(hi, m, kWave));
+            }
+            const float qmax = static_cast<float>((1 << L.bit_v) - 1);
+            const float inv = L.bit_v == 2 ? 1.0f / 3.0f : L.bit_v == 4 ? 1.0f / 15.0f : 1.0f / 255.0f;
+            const float raw = raw_scale(hi, lo, qmax, inv);
+            const float sc = clamp_scale(raw), y = 1.0f / sc;
+            if (!live) continue;
+            int32_t* out = L.v_code + (row0 + tok) * L.v_words + part * L.bit_v;
+            if (L.bit_v == 2) tile_value_words<2>(v, lo, sc, y, raw <= 1e5f, out);
+            else if (L.bit_v == 4) tile_value_words<4>(v, lo, sc, y, raw <= 1e5f, out);
+            else tile_value_words<8>(v, lo, sc, y, raw <= 1e5f, out);
+            if ((part & (group - 1)) == 0) {
+                const int64_t o = (row0 + tok) * L.v_groups + part / group;
+                L.v_scale[o] = f32_to_f16(sc);
+                L.v_min[o] = f32_to_f16(lo);
+            }
+        }
+        return;
+    }
+
+    // ---- Key ----
+    const TileLds tl = tile_lds(L, tb);
+    const CodeSegs cs = code_segs(L);
+    uint8_t* codes = smem;                                   // [tb][ldc], over the staged block
+    uint16_t* kpage = reinterpret_cast<uint16_t*>(smem);     // [tb][D]
+    float2* pmm = reinterpret_cast<float2*>(smem + tl.pmm);  // [tb / 32][D] partial (lo, hi)
+    int16_t* cpos = reinterpret_cast<int16_t*>(smem + tl.cpos);  // code byte of a channel, -1 - rank: fp16 tier
+    int16_t* tidx = reinterpret_cast<int16_t*>(smem + tl.tidx);  // channel of an fp16 slot
+    const int w0 = L.k_width[0], w1 = L.k_width[1], w2 = L.k_width[2], w16 = L.k_width[3];
+    const int n0 = w0 ? L.tier_count[0][h] : 0, n1 = w1 ? L.tier_count[1][h] : 0, n2 = w2 ? L.tier_count[2][h] : 0;
+    const int n3 = w16 ? L.tier_count[3][h] : 0;
+    {
+        const uint16_t* src = static_cast<const uint16_t*>(a.k_src) + off;
+        const int per = D / 8;
+#pragma unroll 4
+        for (int i = tid; i < tb * per; i += kTileThreads) {
+            const int tok = i / per, c = i & (per - 1);
+            reinterpret_cast<uint4*>(kpage)[i] = *reinterpret_cast<const uint4*>(src + tok * a.st + 8 * c);
+        }
+    }
+    const int kg = L.k_group, groups = tb / kg;  // Key groups of the block
+    const int64_t grp0 = (static_cast<int64_t>(page) * L.page_size + t0) / kg;
+    const bool has_sm = L.k_sm_page != nullptr && kg == L.page_size;
+    const SmPage sp = sm_page(L.k_words);
+    uint16_t* smg = has_sm ? L.k_sm_page + sm_page_idx(L, b, h, page) : nullptr;
+    for (int i = tid; i < w0 + w1 + w2 + w16; i += kTileThreads) {
+        const bool in1 = i >= w0, in2 = i >= w0 + w1, in3 = i >= w0 + w1 + w2;
+        const int j = i - pick4(in1, in2, in3, 0, w0, w0 + w1, w0 + w1 + w2);
+        const int32_t* index = pick4(in1, in2, in3, L.tier_index[0], L.tier_index[1], L.tier_index[2], L.tier_index[3]);
+        const int width = pick4(in1, in2, in3, w0, w1, w2, w16);
+        if (j < pick4(in1, in2, in3, n0, n1, n2, n3)) {
+            const int c = index[h * width + j];
+            cpos[c] = static_cast<int16_t>(in3 ? -1 - j : pick3(in1, in2, cs.seg[0], cs.seg[1], cs.seg[2]) + j);
+            if (in3) tidx[j] = static_cast<int16_t>(c);
+        } else if (!in3) {  // padding slots: scale 1.0, min 0.0 (layout.py:84-85)
+            uint16_t* ks = pick3(in1, in2, L.k_scale[0], L.k_scale[1], L.k_scale[2]);
+            uint16_t* km = pick3(in1, in2, L.k_min[0], L.k_min[1], L.k_min[2]);
+            const int64_t o = kgrp_idx(L, b, h, width, j, grp0);
+            for (int g = 0; g < groups; ++g) { ks[o + g] = 0x3C00u; km[o + g] = 0; }
+        }
+    }
+    if (has_sm)
+        for (int p = tid; p < 8 * sp.nb; p += kTileThreads) {
+            const int gb = p >> 3, pos = p & 7;
+            const int t = gb >= sp.blk0[2] ? 2 : gb >= sp.blk0[1] ? 1 : 0;
+            if (sm_slot(t, gb - pick3(t >= 1, t >= 2, 0, sp.blk0[1], sp.blk0[2]), pos) >= pick3(t >= 1, t >= 2, n0, n1, n2)) {
+                smg[16 * gb + pos] = 0x3C00u;
+                smg[16 * gb + 8 + pos] = 0;
+            }
+        }
+    __syncthreads();
+
+    // the thread's pieces: unit u = (channel u % D, tokens 32 (u / D) ..)
+    float x[U][32];
+    const int units = D * tb / 32;
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+        const int u = tid + kTileThreads * k;
+        if (u >= units) continue;
+        const int c = u & (D - 1), ck = u / D;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) x[k][i] = elem_f32<uint16_t, IsHalf>(kpage[(32 * ck + i) * D + c]);
+        float lo, hi;
+        minmax32(x[k], lo, hi);
+        pmm[u] = float2{lo, hi};
+    }
+    if (w16 > 0) {  // fp16 tier, in memory order; padding slots are 0
+        const uint32_t r = __builtin_amdgcn_readfirstlane(tile_rcp(w16));
+        uint16_t* out = L.k_value16 + row0 * w16;
+        for (int i = tid; i < tb * w16; i += kTileThreads) {
+            const int tok = static_cast<int>(i * r >> 20), j = i - tok * w16;
+            out[i] = j < n3 ? f32_to_f16(elem_f32<uint16_t, IsHalf>(kpage[tok * D + tidx[j]])) : static_cast<uint16_t>(0);
+        }
+    }
+    __syncthreads();  // the staged block is dead: the codes may overwrite it
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+        const int u = tid + kTileThreads * k;
+        if (u >= units) continue;
+        const int c = u & (D - 1), ck = u / D;
+        const int pos = cpos[c];
+        if (pos < 0) continue;
+        const int g = 32 * ck / kg;  // the piece's Key group, of pieces g kg / 32 ..
+        float lo = __builtin_inff(), hi = -__builtin_inff();
+        for (int q = g * kg / 32; q < (g + 1) * kg / 32; ++q) {
+            const float2 m = pmm[q * D + c];
+            lo = fminf(lo, m.x);
+            hi = fmaxf(hi, m.y);
+        }
+        const bool in1 = pos >= cs.seg[1], in2 = pos >= cs.seg[2];
+        const float qmax = in2 ? 255.0f : in1 ? 15.0f : 3.0f;
+        const float raw = raw_scale(hi, lo, qmax, in2 ? 1.0f / 255.0f : in1 ? 1.0f / 15.0f : 1.0f / 3.0f);
+        const float sc = clamp_scale(raw), y = 1.0f / sc;
+        if (32 * ck % kg == 0) {
+            const int j = pos - pick3(in1, in2, 0, cs.seg[1], cs.seg[2]);
+            const int64_t o = kgrp_idx(L, b, h, pick3(in1, in2, w0, w1, w2), j, grp0 + g);
+            const uint16_t hs = f32_to_f16(sc), hl = f32_to_f16(lo);
+            pick3(in1, in2, L.k_scale[0], L.k_scale[1], L.k_scale[2])[o] = hs;
+            pick3(in1, in2, L.k_min[0], L.k_min[1], L.k_min[2])[o] = hl;
+            if (has_sm) {
+                int lb, bp;
+                const int t = in2 ? 2 : in1 ? 1 : 0;
+                sm_place(t, j, lb, bp);
+                uint16_t* blk = smg + 16 * (pick3(in1, in2, 0, sp.blk0[1], sp.blk0[2]) + lb);
+                blk[bp] = hs;
+                blk[8 + bp] = hl;
+            }
+        }
+        uint8_t* crow = codes + 32 * ck * tl.ldc + pos;
+        if (raw <= 1e5f) {
+#pragma unroll
+            for (int i = 0; i < 32; ++i) crow[i * tl.ldc] = static_cast<uint8_t>(magic_code(x[k][i], lo, sc, y));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 32; ++i) crow[i * tl.ldc] = static_cast<uint8_t>(fast_code(x[k][i], lo, sc, y, qmax));
+        }
+    }
+    __syncthreads();
+    tile_words<2>(codes, tl.ldc, cs.seg[0], L.k_words[0], n0, tb, L.k_code[0] + row0 * L.k_words[0]);
+    tile_words<4>(codes, tl.ldc, cs.seg[1], L.k_words[1], n1, tb, L.k_code[1] + row0 * L.k_words[1]);
+    tile_words<8>(codes, tl.ldc, cs.seg[2], L.k_words[2], n2, tb, L.k_code[2] + row0 * L.k_words[2]);
+}
+
+// Tokens of a block of the tiled path for this layer and source, or 0 where it does not serve them.
+int pack_tile_tokens(const lf_packed_layer& L, int src_dtype, bool vec16) {
+    const int D = L.head_dim, kg = L.k_group;
+    if (!vec16 || src_dtype == LF_FP32 || (D != 64 && D != 128 && D != 256)) return 0;
+    if (kg % 32 || kg > 128 || L.page_size % kg) return 0;
+    if (L.bit_v < 16 && (L.v_group % 32 || (reinterpret_cast<uintptr_t>(L.v_code) & 7))) return 0;
+    if (L.bit_v >= 16 && (reinterpret_cast<uintptr_t>(L.v_value16) & 3)) return 0;
+    for (int t = 0; t < 3; ++t)
+        if (L.k_words[t] >= 90) return 0;
+    if (L.k_width[3] >= 90) return 0;
+    return kg == 32 && L.page_size % 64 == 0 ? 64 : kg;
+}
+
+template <bool IsHalf>
+int launch_tile(const PackTileArgs& ta, dim3 grid, size_t lds, hipStream_t stream) {
+    const int units = ta.a.L.head_dim * ta.tb / 32, per = (units + kTileThreads - 1) / kTileThreads;
+    auto go = [&](auto kernel) {
+        const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
+        if (rc != LF_OK) return rc;
+        hipLaunchKernelGGL(kernel, grid, dim3(kTileThreads), lds, stream, ta);
+        const hipError_t err = hipGetLastError();
+        return err == hipSuccess ? static_cast<int>(LF_OK) : static_cast<int>(err);
+    };
+    if (per <= 1) return go(pack_tile_kernel<IsHalf, 1>);
+    if (per <= 2) return go(pack_tile_kernel<IsHalf, 2>);
+    return go(pack_tile_kernel<IsHalf, 4>);
+}
+
 int pack_code_row(const lf_packed_layer& L) {
     const int wsum = L.k_width[0] + L.k_width[1] + L.k_width[2];
     return wsum > L.head_dim ? wsum : L.head_dim;
@@ -923,6 +1216,14 @@ int launch_pack_pages(const lf_packed_layer& L, const void* k_src, const void* v
         const dim3 grid2(n_jobs, L.n_kv, 2);  // z: Key page, Value page
         return ld == kCodeLdNarrow ? launch_fast_single<kCodeLdNarrow>(a, half, grid2, lds, stream)
                                    : launch_fast_single<kCodeLdWide>(a, half, grid2, lds, stream);
+    }
+    if (const int tb = pack_tile_tokens(L, src_dtype, a.vec16 != 0)) {
+        const size_t lds = static_cast<size_t>(tile_lds(L, tb).total);
+        if (lds <= 160 * 1024) {
+            const PackTileArgs ta{a, tb};
+            const dim3 tiles(n_jobs, L.n_kv, 2 * (L.page_size / tb));  // z: block of the page, Key and Value
+            return src_dtype == LF_FP16 ? launch_tile<true>(ta, tiles, lds, stream) : launch_tile<false>(ta, tiles, lds, stream);
+        }
     }
     int rc;
     if (src_dtype == LF_BF16) rc = launch_one<uint16_t, false>(a, grid, elem, stream);

@@ -1,0 +1,54 @@
+"""The tiled page packer (pack_tile_kernel) bit-exact against the oracle at the layouts where its
+blocks, pieces and groups change, and for values at the ends of the quantiser's range."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from logitfill_amd.packed import PackedKVManager
+from tests.helpers import assert_history_equal, f32, oracle_store
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,page,kg,vg,bit_v,dtype", [
+    (64, 32, 32, 32, 2, torch.bfloat16),      # one 32-token block, units for half the threads
+    (128, 64, 32, 64, 4, torch.float16),      # two groups a block
+    (128, 128, 32, 32, 8, torch.bfloat16),    # two blocks a page
+    (128, 192, 96, 128, 2, torch.bfloat16),   # groups of three pieces
+    (256, 128, 128, 256, 2, torch.float16),   # four pieces a thread
+    (64, 64, 64, 64, 2, torch.bfloat16),      # the page-major scale copy
+    (128, 128, 128, 128, 16, torch.float16),  # fp16 Values
+])
+def test_tiled_pack_bit_exact(gpu, D, page, kg, vg, bit_v, dtype):
+    rng = np.random.default_rng(D + kg + bit_v)
+    levels = rng.choice(4, size=(2, D), p=[0.5, 0.25, 0.15, 0.1])
+    levels[1] = np.sort(levels[1])            # (heads with other counts: padding slots)
+    g = torch.Generator().manual_seed(page)
+    x = torch.randn(2, 2, 2, 3 * page, D, generator=g)
+    x[0, 0, :, :page] *= 1e-6                 # scales at the lower clamp
+    x[:, 1, 0, page:2 * page] = 0.75          # constant groups
+    x[:, 1, 1, :page] = torch.randint(-8, 9, (page, D), generator=g) * 0.25  # ties
+    if dtype == torch.bfloat16:
+        x[1, 1, 0, 5, 3] = 3e38               # a range past the upper clamp
+        x[1, 0, 1, 7, 2] = -1e6
+    key, value = x[0].to(dtype), x[1].to(dtype)
+    mgr = PackedKVManager([levels], 2, 2, D, page, kg, vg, bit_v, gpu, batch_size=2)
+    mgr.commit(0, key.to(gpu), value.to(gpu))
+    for b in range(2):
+        with np.errstate(over="ignore"):
+            store = oracle_store(levels, f32(key[b]), f32(value[b]), page, kg, vg, bit_v)
+        assert_history_equal(mgr.layers[0], b, store)
+
+
+def test_tiled_scale_copy(gpu):
+    """Where the Key group is the page, the page-major copy holds the reference arrays' values."""
+    levels = np.random.default_rng(5).choice(4, size=(2, 64), p=[0.5, 0.25, 0.15, 0.1])
+    mgr = PackedKVManager([levels], 2, 2, 64, 64, 64, 64, 2, gpu)
+    x = torch.randn(1, 2, 192, 64, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(gpu)
+    mgr.commit(0, x, x)
+    hist_k, _ = mgr.layers[0].export_reference(0)
+    copy = mgr.layers[0].page_scale_copy(0).reshape(2, 3, -1, 2, 8)
+    used = sorted(float(v) for t in range(3) for v in hist_k[t]["scale"].flatten() if v != 1.0)
+    assert used == sorted(float(v) for v in copy[:, :, :, 0].flatten() if v != 1.0)
