@@ -11,11 +11,13 @@
 // takes, with their address, shift, scale and min in registers, so an element costs one 16-bit load
 // (no code crosses 16 bits, and an fp16 value is 16) and its arithmetic, without a branch.  Bound: the float32 writes (8 bytes per token and channel against about one read).
 // The kernel before it looked each element's channel up in the tier tables by a linear scan, V loads
-// and four integer divisions per element: 6 200 tokens x 8 heads x 128 took 279 us, now 25
-// (2 TB/s of writes; about 15 of them are the dependent loads before the first store).
+// and four integer divisions per element: 6 200 tokens x 8 heads x 128 took 279 us, now 26
+// (1.9 TB/s of writes; about 10 of them are the launch and the dependent loads before the first store).
 #pragma clang fp contract(off)
 
-#include "lf_common.hpp"
+#include <algorithm>
+
+#include "decode_common.hpp"
 
 namespace lf {
 namespace {
@@ -28,7 +30,9 @@ struct DequantArgs {
     int both;  // Key and Value: workgroups of each (blockIdx.z & 1)
     float* k_out;
     float* v_out;
+    char pad[96];  // (whole lines for prefetch_args)
 };
+static_assert(sizeof(DequantArgs) > 320 && sizeof(DequantArgs) <= 640, "prefetch_args takes 6 to 10 lines");
 
 constexpr int kThreads = 256;
 constexpr int kSlab = 4096;  // channels of a workgroup (its map: 16 KB of LDS)
@@ -142,6 +146,7 @@ __device__ __forceinline__ void value_rows(const DequantArgs& a, int h, int c, i
 
 template <int V>
 __global__ __launch_bounds__(kThreads) void dequant_kernel(DequantArgs a) {
+    prefetch_args<sizeof(DequantArgs)>();
     extern __shared__ uint32_t map[];  // [channel - c0]: tier << 28 | rank, all ones: no tier
     const lf_packed_layer& L = a.L;
     const int h = blockIdx.y, tid = threadIdx.x;
@@ -162,9 +167,8 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(DequantArgs a) {
             const bool in1 = i >= w0, in2 = i >= w1, in3 = i >= w2;
             const int t = in1 + in2 + in3;
             const int j = i - pick4(in1, in2, in3, 0, w0, w1, w2);
-            if (j >= pick4(in1, in2, in3, n0, n1, n2, n3)) continue;
-            const int c = pick4(in1, in2, in3, i0, i1, i2, i3)[j];
-            if (c >= c0 && c < c0 + D) atomicMin(&map[c - c0], static_cast<uint32_t>(t) << 28 | static_cast<uint32_t>(j));
+            const int c = pick4(in1, in2, in3, i0, i1, i2, i3)[j];  // (with the counts in flight)
+            if (j < pick4(in1, in2, in3, n0, n1, n2, n3) && c >= c0 && c < c0 + D) atomicMin(&map[c - c0], static_cast<uint32_t>(t) << 28 | static_cast<uint32_t>(j));
         }
         __syncthreads();
     }
@@ -187,12 +191,13 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(DequantArgs a) {
 
 int launch_dequantize(const lf_packed_layer& L, int b, int tokens, float* k_out, float* v_out,
                       hipStream_t stream) {
-    // 64 tokens a workgroup, which pays for the tier map, while that leaves four workgroups per CU;
-    // fewer for short histories
-    int run = 64;
-    while (run > 8 && static_cast<int64_t>(tokens) * L.n_kv < 1024LL * run) run /= 2;
+    // As many tokens a workgroup as make two rounds of five workgroups per CU, Key and Value, in
+    // steps of 8, at most 512: one round leaves the last stores without company, more rounds repeat
+    // the dependent loads before a workgroup's first store (us at 2 012 and 6 200 tokens x 8 heads x
+    // 128, runs of 8 and 32: 20.0 and 25.3; of 32 and 80: 15.0 and 27.5; of 16 and 40: 13.9 and 26.3)
+    int run = static_cast<int>(std::min<int64_t>(512, std::max<int64_t>(8, (static_cast<int64_t>(tokens) * L.n_kv * 2 / 2560 + 7) / 8 * 8)));
     while (static_cast<int64_t>(tokens) / run > (1 << 23)) run *= 2;  // the grid's limit
-    DequantArgs a{L, b, tokens, run, k_out && v_out, k_out, v_out};
+    DequantArgs a{L, b, tokens, run, k_out && v_out, k_out, v_out, {}};
     const bool out16 = ((reinterpret_cast<uintptr_t>(k_out) | reinterpret_cast<uintptr_t>(v_out)) & 15) == 0;
     const bool vec = L.head_dim % 4 == 0 && out16 && (!v_out || L.bit_v >= 16 || L.v_group % 4 == 0);
     const dim3 grid((tokens + run - 1) / run, L.n_kv, (L.head_dim + kSlab - 1) / kSlab * (a.both ? 2 : 1));
