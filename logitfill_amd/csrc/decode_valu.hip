@@ -163,7 +163,9 @@ __global__ __launch_bounds__(64) void decode_valu_kernel(DecodeParams p) {
             __syncthreads();
             // Process the group's chunks.
             for (int64_t t0 = tok; t0 < tok + kg; t0 += chunk) {
-                const bool active = lane < chunk;
+                // 64 may not divide the group.
+                const int n_tok = static_cast<int>(min(static_cast<int64_t>(chunk), tok + kg - t0));
+                const bool active = lane < n_tok;
                 const int64_t row = tok_row(L, b, h, t0 + (active ? lane : 0));
                 float score[kMaxG];
 #pragma unroll
@@ -210,7 +212,7 @@ __global__ __launch_bounds__(64) void decode_valu_kernel(DecodeParams p) {
 #pragma unroll
                     for (int i = 0; i < kMaxG; ++i) o[cc][i] *= alpha[i];
                     if (c >= D) continue;
-                    for (int tt = 0; tt < chunk; ++tt) {
+                    for (int tt = 0; tt < n_tok; ++tt) {
                         const uint32_t code = (vcode[tt * vws + (c >> 4)] >> (2 * (c & 15))) & 3u;
                         const float v = static_cast<float>(code) * vsc[tt * vgs + vg] + vmn[tt * vgs + vg];
 #pragma unroll

@@ -107,3 +107,9 @@ def test_tiled_infinite_fp16_key(gpu):
     kn, vn = (torch.randn(1, 1, 1, 64, generator=g).to(gpu) for _ in range(2))
     a, b = (_decode(mgr, q, kn, vn, k) for k in (_native.KERNEL_AUTO, _native.KERNEL_VALU))
     assert torch.isfinite(a).all() and _rel(a, b) < 2e-5
+
+
+def test_general_kernel_group_of_one_and_a_half_chunks(gpu):
+    """Key groups of 96 tokens, which the general kernel's 64-token chunks do not divide."""
+    mgr, _, _, q, kn, vn = _setup(gpu, 128, 96, 96, 64, 12, 2, [11 * 96 + 5, 96], 1, torch.bfloat16)
+    assert _rel(_decode(mgr, q, kn, vn, _native.KERNEL_VALU, 3), _float64(mgr, q, kn, vn)) < 2e-5
