@@ -247,7 +247,10 @@ int64_t lf_decode_workspace_bytes(int32_t n_q, int32_t head_dim, int32_t n_work)
  * device, as the reference falls back to its dense path, reference.py:105-108).  ``kernel``
  * 0 takes the matrix-core kernel where its layout applies (head_dim 128, pages and Key groups
  * of 128 tokens, one Value group per row, some integer Key tier, the page-major Key scale/min
- * copy present, 16-byte aligned rows) and the general VALU kernel otherwise.
+ * copy present, 16-byte aligned rows; many query rows over many pages take a form of it that
+ * unpacks a page once for 128 rows), the tiled matrix-core kernel for head_dim 64, 128 and 256 with
+ * pages and Key groups of whole 32-token pieces, Value groups of 16 * 2^k channels and 16-byte aligned
+ * arrays, and the general VALU kernel otherwise.  ``kernel`` 2 takes the first of these or fails.
  */
 int32_t lf_decode_attention(const lf_packed_layer* layer, const lf_decode_args* args, void* stream);
 

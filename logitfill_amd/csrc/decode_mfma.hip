@@ -5,7 +5,8 @@
 // src/logitfill/packed/kernel.cu:112-190.  Shapes served: head_dim 128,
 // page = Key group = 128 tokens, one Value group per token (v_group 128), int2
 // Values, any number of query rows per kv head ((n_q / n_kv) * q_len, row = head * q_len +
-// token, served 8 rows per workgroup).  Anything else runs the VALU kernel.
+// token, served 8 rows per workgroup; many rows over many pages go to decode_rows.hip, kRowsTiles in
+// decode_common.hpp).  Other layouts run decode_tiled.hip or the VALU kernel.
 //
 // Work: one workgroup of 4 waves per (split item, kv head, tile of 8 query rows); wave w computes
 // tokens 32w..32w+31 (two 16-token tiles) of every page of the item.  Pages arrive by LDS-DMA
@@ -1300,7 +1301,7 @@ __global__ __launch_bounds__(kThreads, 2) void decode_mfma_kernel(MfmaParams mp)
         else residual_mfma<false>(p, b, h, row0, g, rw, tl, qlin, red, wstat, alpha_lds, vst, tid);
     } else if (kind != 0) {
         // ---- residual (kind 1, 2): the tail page and the new token (at most page_size tokens) ----
-        // One new token (q_len 1; the host sends other calls with a residual to the VALU kernel).
+        // One new token (q_len 1; the host sends other calls with a residual to decode_tiled.hip).
         // VALU: wave w scores tokens 32w..32w+31 (lane % 32 = token, lane / 32 = channel half;
         // q read as float4 from LDS), then accumulates them into channels 2*lane, 2*lane+1.
         // One pass, so each wave's max is final.  For 2-byte residual and new-token rows every
