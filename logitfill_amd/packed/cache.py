@@ -227,9 +227,11 @@ class _LayerStore:
         if self._tail_dirty or self._tail_len_dev is None:
             if min(self.tail_lens) == max(self.tail_lens):
                 # one value: a fill in place of the staging and copy, into the tensor that is there
-                # (the decode's argument block keeps its address)
-                if self._tail_len_dev is None:
-                    self._tail_len_dev = torch.empty(self.batch, dtype=torch.int32, device=self.device)
+                # (the decode's argument block keeps its address); one made under inference mode
+                # cannot be written outside of it, so an ordinary tensor takes its place
+                if self._tail_len_dev is None or self._tail_len_dev.is_inference():
+                    with torch.inference_mode(False):
+                        self._tail_len_dev = torch.empty(self.batch, dtype=torch.int32, device=self.device)
                 self._tail_len_dev.fill_(self.tail_lens[0])
             else:
                 self._tail_len_dev = _native.upload(self.tail_lens, torch.int32, self.device)
