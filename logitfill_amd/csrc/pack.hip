@@ -1036,6 +1036,8 @@ __global__ __launch_bounds__(kTileThreads) void pack_tile_kernel(PackTileArgs ta
     const bool has_sm = L.k_sm_page != nullptr && kg == L.page_size;
     const SmPage sp = sm_page(L.k_words);
     uint16_t* smg = has_sm ? L.k_sm_page + sm_page_idx(L, b, h, page) : nullptr;
+    for (int c = tid; c < D; c += kTileThreads) cpos[c] = -1;  // a channel of no tier has no code
+    __syncthreads();
     for (int i = tid; i < w0 + w1 + w2 + w16; i += kTileThreads) {
         const bool in1 = i >= w0, in2 = i >= w0 + w1, in3 = i >= w0 + w1 + w2;
         const int j = i - pick4(in1, in2, in3, 0, w0, w0 + w1, w0 + w1 + w2);
@@ -1219,7 +1221,7 @@ int launch_pack_pages(const lf_packed_layer& L, const void* k_src, const void* v
     }
     if (const int tb = pack_tile_tokens(L, src_dtype, a.vec16 != 0)) {
         const size_t lds = static_cast<size_t>(tile_lds(L, tb).total);
-        if (lds <= 160 * 1024) {
+        if (lds <= 160 * 1024 && 2 * (L.page_size / tb) <= 65535) {
             const PackTileArgs ta{a, tb};
             const dim3 tiles(n_jobs, L.n_kv, 2 * (L.page_size / tb));  // z: block of the page, Key and Value
             return src_dtype == LF_FP16 ? launch_tile<true>(ta, tiles, lds, stream) : launch_tile<false>(ta, tiles, lds, stream);

@@ -52,3 +52,23 @@ def test_tiled_scale_copy(gpu):
     copy = mgr.layers[0].page_scale_copy(0).reshape(2, 3, -1, 2, 8)
     used = sorted(float(v) for t in range(3) for v in hist_k[t]["scale"].flatten() if v != 1.0)
     assert used == sorted(float(v) for v in copy[:, :, :, 0].flatten() if v != 1.0)
+
+
+def test_tiled_pack_channel_of_no_tier(gpu):
+    """Tables that name fewer channels than the head has: the channel left out changes nothing else."""
+    levels = np.random.default_rng(7).choice(4, size=(2, 64), p=[0.5, 0.25, 0.15, 0.1])
+    x = torch.randn(1, 2, 128, 64, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(gpu)
+    full, part = (PackedKVManager([levels], 2, 2, 64, 64, 32, 64, 2, gpu) for _ in range(2))
+    for t in range(4):
+        part.layers[0]._tables_dev[t]["count"].sub_(1)  # every tier's last channel
+    for mgr in (full, part):
+        mgr.commit(0, x, x)
+    (want, want_v), (got, got_v) = (mgr.layers[0].history_views(0) for mgr in (full, part))
+    for name in want_v:
+        assert torch.equal(want_v[name], got_v[name])
+    for t in range(3):
+        for h in range(2):
+            n = int((levels[h] == t).sum()) - 1
+            for name, padding in (("scale", 1.0), ("min", 0.0)):
+                assert torch.equal(want[t][name][h, :n], got[t][name][h, :n])
+                assert bool((got[t][name][h, n].float() == padding).all())
