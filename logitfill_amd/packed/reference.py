@@ -134,12 +134,15 @@ ALONE_FACTOR = 0.78
 
 @functools.lru_cache(maxsize=256)
 def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
-                     overhead: int = ITEM_OVERHEAD_PAGES, per_cu: int = 2) -> int:
+                     overhead: int = ITEM_OVERHEAD_PAGES, per_cu: int = 2, one_round: bool = False) -> int:
     p = np.asarray(pages, dtype=np.int64)
     work = p + residual_pages
     top = max(1, -(-n_kv * int(work.sum()) // slots))
-    # sizes above the one-round size leave slots empty: worth it only when every workgroup then
-    # has a CU to itself
+    # Sizes above the even share leave slots empty: worth it when every workgroup then has a CU to
+    # itself, or when it is what makes one round of ragged sequences whose rounded-up items overflow
+    # the slots at the even share (us per layer-step, two rounds / one: 669 pages in 16 sequences, 4 kv
+    # heads, 4 row tiles, 15- / 34-page items 67.3 / 61.8, 2 tiles, 7 / 15 pages 45.0 / 37.0; 840 in 12, 8
+    # kv heads, 1 tile, 8 / 18 pages 48.0 / 39.6; 40 drawn batches 1.00 to 1.32 times, one 0.98).
     size = np.arange(max(top, int(work.max())), 0, -1, dtype=np.int64)[:, None]   # largest first
     items = np.where(p[None, :] == 0, 1, -(-work[None, :] // size))   # lf_plan_decode's count
     wgs = n_kv * items.sum(axis=1)
@@ -149,12 +152,14 @@ def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
     alone = wgs <= (slots // 2 if per_cu == 2 else 0)
     cost = np.where(alone, (largest + overhead) * ALONE_FACTOR, cost)
     if per_cu == 2:
-        cost = np.where((size[:, 0] > top) & ~alone, np.inf, cost)
+        fits = rounds == 1
+        past = size[:, 0] > top
+        cost = np.where(past & ~alone & ~(one_round & fits & ~np.any(fits & ~past)), np.inf, cost)
     return int(size[int(np.argmin(cost)), 0])                          # ties: fewest items
 
 
 def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int, device=None,
-                           page_elems: int = 128 * 128, per_cu: int = 2) -> int:
+                           page_elems: int = 128 * 128, per_cu: int = 2, one_round: bool = False) -> int:
     """Work per split-K item, in pages.  The decode kernel holds two workgroups per CU (the
     slots).  Items of ``total work / slots`` pages fill the slots once when every sequence's
     work (its pages plus its residual) divides evenly; with ragged lengths the per-sequence
@@ -168,13 +173,14 @@ def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int
     ``ITEM_OVERHEAD_PAGES`` 128 x 128 pages, so smaller pages count more of themselves: 64-token
     pages of head_dim 64 (8 sequences of 50 pages, 2 kv heads) take 4-page items, 15.0 us per
     layer-step, instead of the 2-page ones of an unscaled cost, 18.2.  ``per_cu``: workgroups a
-    CU holds (one of decode_rows.hip)."""
+    CU holds (one of decode_rows.hip).  ``one_round``: sizes above the even share may make the
+    one round that no smaller size does."""
     forced = env_int("LOGITFILL_AMD_PAGES_PER_SPLIT", 0)
     if forced > 0:
         return forced
     slots = per_cu * (_cu_count(device) if device is not None else 256)
     return _pages_per_split(tuple(int(x) for x in hist_pages), int(n_kv), int(residual_pages), slots,
-                            scaled_pages(ITEM_OVERHEAD_PAGES, page_elems), per_cu)
+                            scaled_pages(ITEM_OVERHEAD_PAGES, page_elems), per_cu, bool(one_round))
 
 
 # Of the two decode workgroups that share a CU, the one dispatched second runs this much slower
@@ -471,6 +477,9 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
     # workgroups per (item, kv head): one per tile of query rows
     rows = manager.n_q // manager.n_kv * q_len
     default_layout = P == layer.k_group_size == layer.v_group_size == D == 128
+    # decode_mfma.hip takes the call (fp32 rows of several tokens go to decode_tiled.hip); the other
+    # kernels gain and lose by one-round sizes (0.75 to 1.33 times, 26 layouts and batches)
+    one_round = default_layout and kernel != _native.KERNEL_VALU and (q_len == 1 or query.dtype != torch.float32)
     tiles = -(-rows // MFMA_TILE_ROWS)
     # decode_rows.hip takes the call
     wide = (tiles >= ROWS_TILES and sum(hist_pages) * layer.n_kv * tiles >= ROWS_WORK and default_layout
@@ -484,11 +493,11 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
         # whether the dispatch order of decode_mfma.hip applies (its layout, one row tile): chosen
         # again when one changes
         age = kernel != _native.KERNEL_VALU and tiles == 1 and not wide and default_layout
-        choice_key = (hist_pages, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"), age, tiles, wide)
+        choice_key = (hist_pages, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"), age, tiles, wide, one_round)
         cached = layer.__dict__.get("_lf_split_choice")
         if cached is None or cached[0] != choice_key:
             size = choose_pages_per_split(list(hist_pages), layer.n_kv * tiles, res_pages, layer.device, page_elems,
-                                          1 if wide else 2)
+                                          1 if wide else 2, one_round)
             if age and choice_key[2] is None:
                 cus = _cu_count(layer.device)
                 paired = paired_split(list(hist_pages), layer.n_kv, res_pages, cus, size)

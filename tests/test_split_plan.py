@@ -280,3 +280,25 @@ def test_paired_plan_valid_wherever_chosen():
             assert kinds.count(1) + kinds.count(2) == 1
             assert (kinds.count(1) == 1) == (choice[2] > 0)
     assert chosen > 50
+
+
+@pytest.mark.parametrize("pages,n_kv,res", [
+    ([64, 43, 48, 41, 51, 38, 40, 58, 40, 28, 49, 27, 35, 49, 42, 16], 16, 8),   # four row tiles
+    ([70] * 12, 8, 3), ([93] * 10, 8, 4), ([1], 3, 3), ([0, 0, 5], 8, 3), ([512] * 16, 4, 4), ([1000], 64, 3)])
+def test_one_round_size(pages, n_kv, res, slots=512):
+    """With ``one_round``: a size at or below the even share makes one round, or none does and the
+    choice is either one round or what it was; every sequence keeps its pages."""
+    def workgroups(size):
+        return n_kv * sum(1 if p == 0 else -(-(p + res) // size) for p in pages)
+
+    even = max(1, -(-n_kv * (sum(pages) + res * len(pages)) // slots))
+    before = choose_pages_per_split(pages, n_kv, res)
+    size = choose_pages_per_split(pages, n_kv, res, one_round=True)
+    if any(workgroups(s) <= slots for s in range(1, even + 1)) or size <= even:
+        assert size == before
+    else:
+        assert workgroups(size) <= slots
+    covered = [0] * len(pages)
+    for b, p0, p1, _ in plan_items(pages, size, res):
+        covered[b] += p1 - p0
+    assert covered == list(pages)
