@@ -7,13 +7,19 @@
 //
 // decode_mfma.hip serves 8 rows per workgroup and unpacks every page again for each 8.  Here one
 // workgroup of 8 waves per (split item, kv head, tile of 16 * WR rows) unpacks a page once into LDS
-// as matrix operands -- the Key codes as fp16 integers [token][slot], the Value codes as fp16
-// (code - 1.5) [32 tokens][channel][token], transposed -- and every wave multiplies them with its
-// own 16 rows: WR = 8 row groups, or 4 of them with WT = 2 waves sharing a row group's tokens.  A page's bytes arrive by LDS-DMA, one page ahead of the one being computed.
+// as matrix operands -- the Key codes as fp16 integers and the fp16 tier's values as stored
+// [token][slot], the Value codes as fp16 (code - 1.5) [32 tokens][channel][token], transposed -- and
+// every wave multiplies them with its own 16 rows: WR = 8 row groups, or 4 of them with WT = 2 waves
+// sharing a row group's tokens.  A page's bytes arrive by LDS-DMA, one page ahead of the one being
+// computed.
 //
 // Scores S^T = Codes . Qs^T, Qs = q * (scale * scaling * log2 e) as fp16 hi + lo made in registers
-// from the wave's q (kept packed there); Values O^T = (code - 1.5)^T . P'^T, P' = p * vscale as fp16
-// hi + lo.  A query row is a lane (lane % 16) throughout, so the running max, its rescale and the sums
+// from the wave's q (kept packed there).  Qs carries a power of two per page that brings the largest
+// |q| times the largest scale just below fp16's largest number, so the lo parts stay clear of its
+// smallest (unscaled, an int8 channel's lo lost up to 8e-6 of a score); the sums are divided by it in
+// fp32.  It is never below 1, so Qs holds what decode_mfma.hip's unscaled Qs holds: |q| * scale *
+// scaling * log2 e below 65 504, and no bit fewer.  Values O^T = (code - 1.5)^T . P'^T, P' = p * vscale
+// as fp16 hi + lo, in decode_mfma.hip's range.  A query row is a lane (lane % 16) throughout, so the running max, its rescale and the sums
 // stay in the lane.  The codes enter as they are (decode_mfma.hip adds an offset to each and takes it
 // out of the sums again), so the sums carry no cancelling part.  The tail page and the new tokens
 // follow as dense chunks of 128 tokens through the same buffers.
@@ -21,8 +27,8 @@
 // What bounds it: the LDS reads of the operands (12 of 1 KB per K-step and wave, 5 400 cycles of a
 // page's 15 200 for 128 rows) and the VALU work beside them (Qs 6.5 operations per slot and row, softmax
 // and P' split about 14 per score); the page's unpack takes 2 700.  512 new tokens x 28 q / 4 kv heads
-// over 16 384 tokens: 975 us a layer with decode_mfma.hip's 448 tiles of 8 rows, now 465.  Against
-// float64 (float32 output) 0.2-1.5e-6, decode_mfma.hip 1-6e-5.
+// over 16 384 tokens: 975 us a layer with decode_mfma.hip's 448 tiles of 8 rows, now 473 (470 before the
+// factor of Qs was the page's own).  Against float64 (float32 output) 0.2-1.1e-6, decode_mfma.hip 1-6e-5.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -96,6 +102,33 @@ __device__ __forceinline__ Split2 split2(const float (&x)[8]) {
     return r;
 }
 
+// The largest of x over the wave.
+template <int Ctrl>
+__device__ __forceinline__ float dpp_max(float x) {
+    const int xi = __builtin_bit_cast(int, x);
+    return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(xi, xi, Ctrl, 0xf, 0xf, false)));
+}
+__device__ __forceinline__ float wave_top(float x) {
+    x = dpp_max<0xB1>(x);   // lanes ^ 1
+    x = dpp_max<0x4E>(x);   // ^ 2
+    x = dpp_max<0x141>(x);  // half rows mirrored
+    x = dpp_max<0x140>(x);  // rows mirrored
+    return rows_max(x);
+}
+// Larger 16-bit halves of two words of them (as unsigned numbers).
+__device__ __forceinline__ uint32_t pair_max(uint32_t a, uint32_t b) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
+// Exponent of a page's factor on Qs: brings ``top`` (kTopMargin times a bound of |Qs|) into [2^15, 2^16),
+// the bound itself then below 65 504; none below 1, and none past 2^24 (tiny or no q).
+constexpr float kTopMargin = 1.001f;
+__device__ __forceinline__ int qs_exponent(float top) {
+    return min(max(142 - static_cast<int>(__float_as_uint(top) >> 23), 0), 24);
+}
+__device__ __forceinline__ float exp_of_2(int k) { return __uint_as_float(static_cast<uint32_t>(127 + k) << 23); }
+
 template <bool Bf>
 __device__ __forceinline__ float4v mfma16(u32x4 a, u32x4 b, float4v c) {
     if constexpr (Bf) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -137,7 +170,8 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
     unsigned char* kbuf = smem;
     unsigned char* vbuf = smem + y.off_v;
     float* sbuf = reinterpret_cast<float*>(smem + y.off_s);  // Key scales [nb * 8], mins [nb * 8]
-    float* vsb = sbuf + 16 * y.nb;                            // Value scales [128], scaled middles [128]
+    float* vsb = sbuf + 16 * y.nb;                            // Value scales [128], scaled middles [128],
+                                                              // 1 / the page's factor
 
     const uint16_t* qrow = static_cast<const uint16_t*>(A.query) + (static_cast<int64_t>(b) * A.n_q + h * p.g + row_safe) * kD;
     auto widen = [](uint32_t u) { return Bf ? bf16_to_f32(static_cast<uint16_t>(u)) : f16_to_f32(static_cast<uint16_t>(u)); };
@@ -182,11 +216,19 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
         // position and row took the prologue 18 us).
         constexpr int kQStride = 2 * kD + 16;
         int16_t* chan = reinterpret_cast<int16_t*>(vbuf);
+        uint32_t qtop = 0;  // largest |q| bits of the thread's elements, even and odd ones
         for (int i = tid; i < 16 * kWR * 16; i += kThreads) {
             const int r = min(row_first + (i >> 4), p.g - 1);
-            *reinterpret_cast<u32x4*>(kbuf + (i >> 4) * kQStride + 16 * (i & 15)) = *reinterpret_cast<const u32x4*>(
+            const u32x4 q = *reinterpret_cast<const u32x4*>(
                 static_cast<const uint16_t*>(A.query) + (static_cast<int64_t>(b) * A.n_q + h * p.g + r) * kD + 8 * (i & 15));
+            *reinterpret_cast<u32x4*>(kbuf + (i >> 4) * kQStride + 16 * (i & 15)) = q;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) qtop = pair_max(qtop, q[k] & 0x7fff7fffu);
         }
+        // (a NaN counts as an infinity: the factor is then 1 and the bound holds for the other rows)
+        qtop = max(qtop & 0xffffu, qtop >> 16);
+        const float top = wave_top(fminf(fabsf(widen(qtop)), __builtin_inff()));
+        if (lane == 0) vsb[wave] = top;
         if (tid < 8 * y.nb) {
             const int s = tid >> 5;
             const bool in1 = s >= st1, in2 = s >= st2, in3 = s >= st3;
@@ -196,6 +238,10 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
             chan[tid] = static_cast<int16_t>(c);
         }
         __syncthreads();
+        float qbound = vsb[0];
+#pragma unroll
+        for (int k = 1; k < kWaves; ++k) qbound = fmaxf(qbound, vsb[k]);
+        qbound *= fabsf(p.qscale) * kTopMargin;  // of |Qs| / scale
         u32x4 qr[kMaxSteps];
 #pragma unroll
         for (int s = 0; s < kMaxSteps; ++s) {
@@ -253,6 +299,27 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
         auto unpack_page = [&](const unsigned char* raw) {
             // (fresh: addresses are computed here, not kept in registers over the page loop)
             const int tid = static_cast<int>(fresh(threadIdx.x));
+            // Scales and mins: every wave that needs the page's largest scale (1 for the fp16 tier) finds
+            // it itself
+            if (__builtin_amdgcn_readfirstlane(tid) < 8 * y.nb) {
+                const unsigned char* sm = raw + 16 * e6;
+                uint32_t t2 = w16 > 0 ? 0x3C00u : 0u;
+                if (lane < y.nb_int) {
+                    const u32x4 w = *reinterpret_cast<const u32x4*>(sm + 32 * lane);
+                    t2 = pair_max(pair_max(t2, w[0]), pair_max(w[1], pair_max(w[2], w[3])));
+                }
+                const float top = wave_top(f16_to_f32(static_cast<uint16_t>(max(t2 & 0xffffu, t2 >> 16)))) * qbound;
+                const int k = qs_exponent(top);
+                const float unit = p.qscale * exp_of_2(k);
+                if (tid < 8 * y.nb_int) {
+                    const uint16_t* at = reinterpret_cast<const uint16_t*>(sm) + (tid >> 3) * 16 + (tid & 7);
+                    sbuf[tid] = f16_to_f32(at[0]) * unit;
+                    sbuf[8 * y.nb + tid] = f16_to_f32(at[8]) * p.qscale;
+                } else if (tid < 8 * y.nb) {  // (their mins stay 0)
+                    sbuf[tid] = unit;
+                }
+                if (tid == 0) vsb[2 * kPage] = exp_of_2(-k);
+            }
             for (int c = tid; c < e3; c += kThreads) {
                 const u32x4 w4 = *reinterpret_cast<const u32x4*>(raw + 16 * c);
                 if (c < e0) {  // int2: 16 codes a word, block halves (j, j + 8), j = 0..3 and 4..7
@@ -266,15 +333,12 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
                                                                       code_pair(w >> 4, key_table, pairs, zero), code_pair(w >> 6, key_table, pairs, zero));
                     }
                 } else if (c < e2) {
-                    // int4 as code / 4, int8 as code / 64: the code's bits under the exponent of 256
-                    // or 16, less that (exact).  Their scales carry the factor, so every tier's Qs
-                    // spans what int2's does and its lo part stays clear of fp16's smallest numbers
-                    // (unscaled, the int8 tier's lo lost up to 8e-6 of a score per channel).
+                    // int4 and int8: the code's bits under the exponent of 1 024, less that (exact)
                     const bool four = c < e1;
                     const uint32_t words = four ? w1 : w2, rec_w = four ? r1 : r2;
-                    auto ints = [&](uint32_t x, uint32_t mask) {
-                        const _Float16 z = static_cast<_Float16>(four ? 256.f : 16.f);
-                        return __builtin_bit_cast(half2v, (x & mask) | (four ? 0x5C005C00u : 0x4C004C00u)) - half2v{z, z};
+                    auto ints = [](uint32_t x, uint32_t mask) {
+                        const _Float16 z = static_cast<_Float16>(1024.f);
+                        return __builtin_bit_cast(half2v, (x & mask) | 0x64006400u) - half2v{z, z};
                     };
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
@@ -293,12 +357,11 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
                         }
                     }
                 } else {
-                    // the fp16 value / 64, its q times 64 (as the int8 tier's)
 #pragma unroll
                     for (int k = 0; k < 8; ++k) {
                         const uint32_t idx = 8 * (c - e2) + k, tok = idx * r16 >> 20, j = idx - tok * w16;
-                        *reinterpret_cast<_Float16*>(kbuf + tok * stride + 4 * st3 * 16 + j * 2) =
-                            __builtin_bit_cast(_Float16, static_cast<uint16_t>(w4[k >> 1] >> (16 * (k & 1)))) * static_cast<_Float16>(0.015625f);
+                        *reinterpret_cast<uint16_t*>(kbuf + tok * stride + 4 * st3 * 16 + j * 2) =
+                            static_cast<uint16_t>(w4[k >> 1] >> (16 * (k & 1)));
                     }
                 }
             }
@@ -319,12 +382,6 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
                 *reinterpret_cast<half8*>(vbuf + vt_at(oct >> 2, 16 * word + 4 * by + j, oct & 3)) =
                     as_half8(code_pair(pr[0] >> (2 * j), value_table, pairs, zero), code_pair(pr[1] >> (2 * j), value_table, pairs, zero),
                              code_pair(pr[2] >> (2 * j), value_table, pairs, zero), code_pair(pr[3] >> (2 * j), value_table, pairs, zero));
-            if (tid < 8 * y.nb_int) {
-                const uint16_t* sm = reinterpret_cast<const uint16_t*>(raw + 16 * e6) + (tid >> 3) * 16 + (tid & 7);
-                const float unit = (tid >> 3) >= 4 * st2 ? 64.f : (tid >> 3) >= 4 * st1 ? 4.f : 1.f;
-                sbuf[tid] = f16_to_f32(sm[0]) * p.qscale * unit;
-                sbuf[8 * y.nb + tid] = f16_to_f32(sm[8]) * p.qscale;
-            }
             if (tid < kPage) {
                 const float s = f16_to_f32(reinterpret_cast<const uint16_t*>(raw + 16 * e4)[tid]);
                 vsb[tid] = s;
@@ -332,12 +389,9 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
             }
         };
 
-        // blocks of padding words stay 0; the fp16 tier's scale is 64 (its values come divided by it)
+        // blocks of padding words stay 0, as do the fp16 tier's mins
         for (int i = tid; i < kPage * y.stride / 16; i += kThreads) reinterpret_cast<u32x4*>(kbuf)[i] = u32x4{0, 0, 0, 0};
-        for (int i = 8 * y.nb_int + tid; i < 8 * y.nb; i += kThreads) {
-            sbuf[i] = 64.f * p.qscale;
-            sbuf[8 * y.nb + i] = 0.f;
-        }
+        for (int i = 8 * y.nb_int + tid; i < 8 * y.nb; i += kThreads) sbuf[8 * y.nb + i] = 0.f;
         load_page(0);
         for (int page = pbeg; page < pend; ++page) {
             const int buffer = (page - pbeg) & 1;
@@ -353,9 +407,12 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
             for (int T = 0; T < kTT; ++T) acc[T] = float4v{0.f, 0.f, 0.f, 0.f};
             float bias = 0.f;
             const unsigned char* krow = kbuf + (16 * kTT * wt + n) * stride + q4 * 16;
+            // (the count is laundered: ten conditions kept over the page loop cost SGPR spills)
+            int n_steps = steps;
+            asm volatile("" : "+s"(n_steps));
 #pragma unroll
             for (int s = 0; s < kMaxSteps; ++s) {
-                if (s >= steps) continue;
+                if (s >= n_steps) continue;
                 const float4v* sp = reinterpret_cast<const float4v*>(sbuf + (4 * s + q4) * 8);
                 const float4v* mp = reinterpret_cast<const float4v*>(sbuf + 8 * y.nb + (4 * s + q4) * 8);
                 const float4v sa = sp[0], sb = sp[1], ma = mp[0], mb = mp[1];
@@ -375,10 +432,11 @@ __global__ __launch_bounds__(kThreads, 2) void decode_rows_kernel(RowsParams rp)
 #pragma unroll
                 for (int T = 0; T < kTT; ++T) acc[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[T], B.hi, acc[T], 0, 0, 0);
             }
+            const float inv = vsb[2 * kPage];
             bias = rows_sum(bias);
             float s[kTT * 4];
 #pragma unroll
-            for (int e = 0; e < kTT * 4; ++e) s[e] = acc[e >> 2][e & 3] + bias;
+            for (int e = 0; e < kTT * 4; ++e) s[e] = fmaf(acc[e >> 2][e & 3], inv, bias);
             softmax(s);
 
             // ---- Values ----
@@ -581,7 +639,7 @@ bool plan_rows(const lf_packed_layer& L, RowsLayout& y) {
         c += i < 3 ? kPage / 4 * L.k_words[i] : i == 3 ? kPage / 8 * L.k_width[3] : i == 4 ? kPage * 2 : i < 7 ? kPage / 8 : 2 * y.nb_int;
         y.end[i] = c;
     }
-    if (c > 64 * kWaves * kMaxDma || 8 * y.nb_int > kThreads) return false;
+    if (c > 64 * kWaves * kMaxDma || 8 * y.nb > kThreads) return false;
     for (int t = 0; t < 3; ++t)
         if (L.k_width[t] && (!aligned(L.k_code[t], 16) || L.k_words[t] >= 90)) return false;
     if (L.k_width[3] && (!aligned(L.k_value16, 16) || L.k_width[3] >= 90)) return false;
@@ -590,7 +648,7 @@ bool plan_rows(const lf_packed_layer& L, RowsLayout& y) {
     y.stride = 16 * y.nb + 16;
     y.off_v = kPage * std::max(y.stride, kDenseStride);
     y.off_s = y.off_v + kVtBytes;
-    y.off_raw = y.off_s + (16 * y.nb + 2 * kPage) * 4;
+    y.off_raw = y.off_s + (16 * y.nb + 2 * kPage + 4) * 4;
     y.raw_bytes = 1024 * ((c + 63) / 64);
     y.lds_bytes = y.off_raw + 2 * y.raw_bytes;
     const int merge = kWaves * 16 * (kD + 4) * 4 + 2 * kWaves * 16 * 4;

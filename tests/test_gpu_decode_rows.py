@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from logitfill_amd import _native
+from logitfill_amd.packed import PackedKVManager
 from logitfill_amd.packed.reference import decode_into
 from tests.test_gpu_tiled import _decode, _float64, _rel, _setup
 
@@ -50,3 +51,50 @@ def test_many_rows_commit(gpu):
     tk, tv = layer.tail_buffers()
     assert layer.tail_lens == [29] and layer.tail_len_device().tolist() == [29]
     assert torch.equal(tk[:, :, 17:29], kn) and torch.equal(tv[:, :, 17:29], vn)
+
+
+# Eight channels of a tier of their own: (tier, Key sigma, q of every second row there, scaling).
+RANGES = {
+    "fp16_keys_1e-3": (3, 1e-3, 4e3, None),      # stored values below 2^-8
+    "fp16_keys_1e-4": (3, 1e-4, 5e3, None),
+    "fp16_large_q": (3, 1e-3, 3e4, None),
+    "fp16_scaling_1": (3, 1e-2, 800.0, 1.0),
+    "int8_large_q": (2, 2e3, 1500.0, None),      # |q| x scale about 65 000
+    "int4_large_q": (1, 1e4, 60.0, None),        # ... 300 000
+    "plain": (2, 1.0, 0.1, None),
+}
+
+
+@pytest.mark.parametrize("name", RANGES)
+def test_many_rows_operand_range(gpu, name):
+    """Small fp16-tier Keys keep their bits and large q stay finite, as in decode_mfma.hip: no row
+    further from float64 than twice that kernel's furthest on the same call (both sum in float32, in
+    another order), plus 2e-6 for the float32 spacing of the scores.  (An overflow leaves a row empty or
+    NaN: a distance of 1 or none.)"""
+    tier, sigma, level, scaling = RANGES[name]
+    scaling = 128 ** -0.5 if scaling is None else scaling
+    n_q, T = 48, 505 * 128 + 20
+    rng = np.random.default_rng(11)
+    levels = np.where(rng.random((1, 128)) < 0.3, 1, 0)
+    special = rng.permutation(128)[:8]
+    levels[0, special] = tier
+    g = torch.Generator().manual_seed(11)
+    key, value = (torch.randn(1, 1, T, 128, generator=g) for _ in range(2))
+    key[..., special] *= sigma
+    q = torch.randn(1, n_q, 1, 128, generator=g) * 128 ** -0.5
+    q[:, ::2, :, special] = level * (0.5 + torch.rand(1, n_q // 2, 1, 8, generator=g))
+    kn, vn = (torch.randn(1, 1, 1, 128, generator=g) for _ in range(2))
+    key, value, q, kn, vn = (t.to(torch.float16).to(gpu) for t in (key, value, q, kn, vn))
+    mgr = PackedKVManager([levels], n_q, 1, 128, 128, 128, 128, 2, gpu)
+    mgr.commit(0, key, value)
+    want = _float64(mgr, q.double() * (scaling * 128 ** 0.5), kn, vn)
+
+    def furthest(kernel):
+        out = torch.empty(q.shape, dtype=torch.float32, device=gpu)
+        decode_into(mgr, 0, q, kn, vn, scaling, out, kernel=kernel)
+        torch.cuda.synchronize()
+        return float(((out.double() - want).norm(dim=-1) / want.norm(dim=-1)).max())
+
+    wide, narrow = furthest(_native.KERNEL_AUTO), furthest(_native.KERNEL_MFMA)
+    print(f"{name}: many rows {wide:.2e} decode_mfma {narrow:.2e}")
+    assert narrow < 1e-2 and wide < 2 * narrow + 2e-6
