@@ -920,6 +920,17 @@ __device__ __forceinline__ void tile_words(const uint8_t* codes, int ldc, int se
     }
 }
 
+// raw_scale and fast_code with the general kernel's bytes for what their clamp to FLT_MAX hides: a range
+// of inf - inf (every element the same infinity) takes the smallest scale, a NaN or -inf - -inf code 0.
+__device__ __forceinline__ float tile_raw_scale(float hi, float lo, float qmax, float inv) {
+    const float range = hi - lo;
+    return range != range ? range : raw_scale(hi, lo, qmax, inv);
+}
+__device__ __forceinline__ uint32_t tile_code(float x, float lo, float s, float y, float qmax) {
+    const float a = x - lo;
+    return a != a ? 0u : fast_code(x, lo, s, y, qmax);
+}
+
 // 32 channels of a token, Bits per code, into out (Bits words).
 template <int Bits>
 __device__ __forceinline__ void tile_value_words(const float (&v)[32], float lo, float sc, float y, bool magic, int32_t* out) {
@@ -932,7 +943,7 @@ __device__ __forceinline__ void tile_value_words(const float (&v)[32], float lo,
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const float x = v[kPer * j + i];
-            const uint32_t code = magic ? magic_code(x, lo, sc, y) & 0xffu : fast_code(x, lo, sc, y, kQmax);
+            const uint32_t code = magic ? magic_code(x, lo, sc, y) & 0xffu : tile_code(x, lo, sc, y, kQmax);
             w[j] |= code << (Bits * i);
         }
     }
@@ -993,9 +1004,11 @@ __global__ __launch_bounds__(kTileThreads) void pack_tile_kernel(PackTileArgs ta
                 lo = fminf(lo, __shfl_xor(lo, m, kWave));
                 hi = fmaxf(hi, __shfl_xor(hi, m, kWave));
             }
+            lo = fminf(lo, __builtin_inff());  // (a group of NaN alone)
+            hi = fmaxf(hi, -__builtin_inff());
             const float qmax = static_cast<float>((1 << L.bit_v) - 1);
             const float inv = L.bit_v == 2 ? 1.0f / 3.0f : L.bit_v == 4 ? 1.0f / 15.0f : 1.0f / 255.0f;
-            const float raw = raw_scale(hi, lo, qmax, inv);
+            const float raw = tile_raw_scale(hi, lo, qmax, inv);
             const float sc = clamp_scale(raw), y = 1.0f / sc;
             if (!live) continue;
             int32_t* out = L.v_code + (row0 + tok) * L.v_words + part * L.bit_v;
@@ -1104,7 +1117,7 @@ __global__ __launch_bounds__(kTileThreads) void pack_tile_kernel(PackTileArgs ta
         }
         const bool in1 = pos >= cs.seg[1], in2 = pos >= cs.seg[2];
         const float qmax = in2 ? 255.0f : in1 ? 15.0f : 3.0f;
-        const float raw = raw_scale(hi, lo, qmax, in2 ? 1.0f / 255.0f : in1 ? 1.0f / 15.0f : 1.0f / 3.0f);
+        const float raw = tile_raw_scale(hi, lo, qmax, in2 ? 1.0f / 255.0f : in1 ? 1.0f / 15.0f : 1.0f / 3.0f);
         const float sc = clamp_scale(raw), y = 1.0f / sc;
         if (32 * ck % kg == 0) {
             const int j = pos - pick3(in1, in2, 0, cs.seg[1], cs.seg[2]);
@@ -1127,7 +1140,7 @@ __global__ __launch_bounds__(kTileThreads) void pack_tile_kernel(PackTileArgs ta
             for (int i = 0; i < 32; ++i) crow[i * tl.ldc] = static_cast<uint8_t>(magic_code(x[k][i], lo, sc, y));
         } else {
 #pragma unroll
-            for (int i = 0; i < 32; ++i) crow[i * tl.ldc] = static_cast<uint8_t>(fast_code(x[k][i], lo, sc, y, qmax));
+            for (int i = 0; i < 32; ++i) crow[i * tl.ldc] = static_cast<uint8_t>(tile_code(x[k][i], lo, sc, y, qmax));
         }
     }
     __syncthreads();

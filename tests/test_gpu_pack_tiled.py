@@ -72,3 +72,41 @@ def test_tiled_pack_channel_of_no_tier(gpu):
             for name, padding in (("scale", 1.0), ("min", 0.0)):
                 assert torch.equal(want[t][name][h, :n], got[t][name][h, :n])
                 assert bool((got[t][name][h, n].float() == padding).all())
+
+
+@pytest.mark.parametrize("D,page,kg,vg,bit_v,dtype", [
+    (64, 64, 32, 32, 2, torch.bfloat16),
+    (128, 64, 64, 64, 4, torch.float16),
+    (128, 96, 96, 32, 8, torch.bfloat16),
+])
+def test_tiled_pack_not_finite(gpu, D, page, kg, vg, bit_v, dtype):
+    """Infinities and NaN: the bytes are those of the general packer, which float32 pages of the same
+    values take."""
+    levels = np.random.default_rng(D + kg).choice(4, size=(2, D), p=[0.4, 0.3, 0.2, 0.1])
+    g = torch.Generator().manual_seed(kg)
+    x = torch.randn(2, 1, 2, 3 * page, D, generator=g)
+    inf, nan = float("inf"), float("nan")
+    x[:, 0, 0, 3, ::3] = inf                 # one infinity in a group, of either sign
+    x[:, 0, 0, 7, 1::3] = -inf
+    x[:, 0, 0, page:page + kg, 5:40] = inf   # whole groups of one infinity
+    x[:, 0, 1, page:page + kg, 5:40] = -inf
+    x[:, 0, 1, 4, :] = nan                   # a NaN among finite values, among a large range, alone
+    x[:, 0, 1, 5, ::2] = 6e4
+    x[:, 0, 1, 6, ::2] = -6e4
+    x[:, 0, 0, 2 * page:2 * page + kg, 2:36] = nan
+    key, value = x[0].to(dtype).to(gpu), x[1].to(dtype).to(gpu)
+    mgr, general = (PackedKVManager([levels], 2, 2, D, page, kg, vg, bit_v, gpu) for _ in range(2))
+    mgr.commit(0, key, value)
+    general.commit(0, key.float(), value.float())
+    (hk, hv), (gk, gv) = (m.layers[0].export_reference(0) for m in (mgr, general))
+    for t in range(4):
+        for name in hk[t]:
+            same = hk[t][name].view(torch.int16) == gk[t][name].view(torch.int16)
+            if hk[t][name].dtype == torch.float16:  # (a NaN's payload may differ between the types)
+                same |= hk[t][name].isnan() & gk[t][name].isnan()
+            assert bool(same.all()), (t, name)
+    for name in hv:
+        same = hv[name].view(torch.int16) == gv[name].view(torch.int16)
+        if hv[name].dtype == torch.float16:
+            same |= hv[name].isnan() & gv[name].isnan()
+        assert bool(same.all()), name
