@@ -255,6 +255,19 @@ int64_t lf_decode_workspace_bytes(int32_t n_q, int32_t head_dim, int32_t n_work)
 int32_t lf_decode_attention(const lf_packed_layer* layer, const lf_decode_args* args, void* stream);
 
 /*
+ * The kernel lf_decode_attention takes for this call (host function, no device access): an LF_KERNEL_*
+ * value or a negative LF_E_*.  For a caller that sizes its work plan for the kernel, so the plan's fields
+ * (work, n_work, seq_work, their host copies, workspace, out, tail_len) may be empty; ``pages`` is the
+ * number of packed pages of the whole batch.  A plan given without work_host keeps LF_KERNEL_ROWS from
+ * being taken, one of more than 65535 items LF_KERNEL_ROWS and LF_KERNEL_TILED.
+ */
+#define LF_KERNEL_VALU 1
+#define LF_KERNEL_MFMA 2
+#define LF_KERNEL_ROWS 3   /* many query rows: pages unpacked once for 64 or 128 of them */
+#define LF_KERNEL_TILED 4  /* the other layouts on the matrix cores */
+int32_t lf_decode_kernel(const lf_packed_layer* layer, const lf_decode_args* args, int64_t pages);
+
+/*
  * Decode attention that allocates nothing (no counterpart in the reference): for callers
  * that cannot allocate device memory -- code under HIP graph capture, tight serving loops,
  * harnesses that forbid allocation.  Same arguments, checks, kernels and results as

@@ -16,6 +16,8 @@ LIB_PATH = Path(__file__).resolve().with_name("liblogitfill_amd.so")
 LF_BF16, LF_FP16, LF_FP32 = 0, 1, 2
 LF_OK, LF_E_NULL, LF_E_SHAPE, LF_E_UNSUPPORTED, LF_E_WORKSPACE, LF_E_DTYPE = 0, -1, -2, -3, -4, -5
 KERNEL_AUTO, KERNEL_VALU, KERNEL_MFMA = 0, 1, 2
+# the kernels a call can take (lf_decode_kernel)
+KERNEL_ROWS, KERNEL_TILED = 3, 4
 
 
 class NativeLibraryMissing(RuntimeError):
@@ -102,6 +104,7 @@ _SIGNATURES = {
     "lf_plan_decode": (c_int32, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_int32, c_void_p]),
     "lf_decode_workspace_bytes": (c_int64, [c_int32, c_int32, c_int32]),
     "lf_decode_attention": (c_int32, [POINTER(PackedLayer), POINTER(DecodeArgs), c_void_p]),
+    "lf_decode_kernel": (c_int32, [POINTER(PackedLayer), POINTER(DecodeArgs), c_int64]),
     "lf_dequantize": (c_int32, [POINTER(PackedLayer), c_int32, c_int32, c_void_p, c_void_p, c_void_p]),
     "lf_dense_decode_workspace_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32]),
     "lf_dense_decode": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,

@@ -80,15 +80,8 @@ int32_t check_layer(const lf_packed_layer* L, bool need_k = true, bool need_v = 
 
 namespace lf {
 
-// Checks shared by the decode entry points, then the launch with ``workspace`` (at least
-// ``workspace_bytes``) as the split-K partials.  The args' own workspace fields are not read.
-int32_t decode_checked(const lf_packed_layer* layer, const lf_decode_args* args, void* workspace,
-                       int64_t workspace_bytes, void* stream) {
-    const int32_t st = check_layer(layer);
-    if (st != LF_OK) return st;
-    if (!args) return LF_E_NULL;
-    const lf_decode_args& A = *args;
-    if (!A.query || !A.out || !A.work || !A.seq_work || !workspace || !A.tail_len) return LF_E_NULL;
+// Shapes, types and rows of a decode call, into ``p`` (its plan and workspace are not looked at).
+int32_t decode_shape(const lf_packed_layer* layer, const lf_decode_args& A, DecodeParams& p) {
     if ((A.k_new == nullptr) != (A.v_new == nullptr)) return LF_E_NULL;
     if (!valid_dtype(A.q_dtype) || !valid_dtype(A.out_dtype) || !valid_dtype(A.tail_dtype)) return LF_E_DTYPE;
     if (A.k_new && !valid_dtype(A.new_dtype)) return LF_E_DTYPE;
@@ -98,31 +91,44 @@ int32_t decode_checked(const lf_packed_layer* layer, const lf_decode_args* args,
     // q_len new tokens: the kernels serve n_q * q_len query rows (row = head * q_len + token)
     const int64_t rows = static_cast<int64_t>(A.n_q) * q_len;
     if (rows > (1 << 20)) return LF_E_SHAPE;
-    // rows per kv head: any number (the kernels tile them across workgroups)
-    const int g = static_cast<int>(rows / layer->n_kv);
     if (layer->bit_v != 2) return LF_E_UNSUPPORTED;  // as reference.py:62
     const int D = layer->head_dim;
     if (D < 8 || D > 1024 || (D & (D - 1)) != 0) return LF_E_UNSUPPORTED;  // as kernel.cu:224-230
     if (layer->v_groups > 64) return LF_E_UNSUPPORTED;
     if (A.tail_cap < 0 || A.tail_cap > layer->page_size) return LF_E_SHAPE;
     if (A.tail_cap > 0 && (!A.tail_k || !A.tail_v)) return LF_E_NULL;
-    if (A.n_work <= 0 || static_cast<int64_t>(A.n_work) * layer->n_kv > 0x7fffffff) return LF_E_SHAPE;
-    if (workspace_bytes < lf_decode_workspace_bytes(static_cast<int32_t>(rows), D, A.n_work)) return LF_E_WORKSPACE;
-    if (A.kernel < 0 || A.kernel > 2) return LF_E_SHAPE;
-    if (A.commit_new != 0 && A.commit_new != 1) return LF_E_SHAPE;
-    if (A.commit_new && (!A.k_new || A.tail_cap < q_len)) return LF_E_SHAPE;  // rows to append, room for them
-
-    DecodeParams p;
     p.L = *layer;
     p.A = A;
     p.A.n_q = static_cast<int32_t>(rows);
-    p.A.workspace = workspace;
-    p.A.workspace_bytes = workspace_bytes;
-    p.g = g;
+    // rows per kv head: any number (the kernels tile them across workgroups)
+    p.g = static_cast<int>(rows / layer->n_kv);
     p.q_len = q_len;
     p.qscale = A.scaling * kLog2e;
-    p.part = static_cast<float*>(workspace);
     p.dense_splits = 0;
+    return LF_OK;
+}
+
+// Checks shared by the decode entry points, then the launch with ``workspace`` (at least
+// ``workspace_bytes``) as the split-K partials.  The args' own workspace fields are not read.
+int32_t decode_checked(const lf_packed_layer* layer, const lf_decode_args* args, void* workspace,
+                       int64_t workspace_bytes, void* stream) {
+    const int32_t st = check_layer(layer);
+    if (st != LF_OK) return st;
+    if (!args) return LF_E_NULL;
+    const lf_decode_args& A = *args;
+    if (!A.query || !A.out || !A.work || !A.seq_work || !workspace || !A.tail_len) return LF_E_NULL;
+    DecodeParams p;
+    const int32_t shape = decode_shape(layer, A, p);
+    if (shape != LF_OK) return shape;
+    if (A.n_work <= 0 || static_cast<int64_t>(A.n_work) * layer->n_kv > 0x7fffffff) return LF_E_SHAPE;
+    if (workspace_bytes < lf_decode_workspace_bytes(p.A.n_q, layer->head_dim, A.n_work)) return LF_E_WORKSPACE;
+    if (A.kernel < 0 || A.kernel > 2) return LF_E_SHAPE;
+    if (A.commit_new != 0 && A.commit_new != 1) return LF_E_SHAPE;
+    if (A.commit_new && (!A.k_new || A.tail_cap < p.q_len)) return LF_E_SHAPE;  // rows to append, room for them
+
+    p.A.workspace = workspace;
+    p.A.workspace_bytes = workspace_bytes;
+    p.part = static_cast<float*>(workspace);
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (A.kernel != 1) {
         bool handled = false;
@@ -233,6 +239,21 @@ int64_t lf_decode_workspace_bytes(int32_t n_q, int32_t head_dim, int32_t n_work)
 int32_t lf_decode_attention(const lf_packed_layer* layer, const lf_decode_args* args, void* stream) {
     return lf::decode_checked(layer, args, args ? args->workspace : nullptr, args ? args->workspace_bytes : 0,
                               stream);
+}
+
+int32_t lf_decode_kernel(const lf_packed_layer* layer, const lf_decode_args* args, int64_t pages) {
+    const int32_t st = check_layer(layer);
+    if (st != LF_OK) return st;
+    if (!args || !args->query) return LF_E_NULL;
+    if (args->kernel < 0 || args->kernel > 2 || pages < 0) return LF_E_SHAPE;
+    lf::DecodeParams p;
+    const int32_t shape = lf::decode_shape(layer, *args, p);
+    if (shape != LF_OK) return shape;
+    if (args->kernel == LF_KERNEL_VALU) return LF_KERNEL_VALU;
+    if (args->kernel == 0 && lf::decode_rows_serves(p, pages)) return LF_KERNEL_ROWS;
+    if (lf::decode_mfma_serves(p)) return LF_KERNEL_MFMA;
+    if (args->kernel == LF_KERNEL_MFMA) return LF_E_UNSUPPORTED;
+    return lf::decode_tiled_serves(p) ? LF_KERNEL_TILED : LF_KERNEL_VALU;
 }
 
 int32_t lf_dequantize(const lf_packed_layer* layer, int32_t b, int32_t tokens, float* k_out, float* v_out,

@@ -209,6 +209,12 @@ __device__ __forceinline__ void commit_new_rows(const DecodeParams& p, int b, in
 constexpr int kRowsTiles = 6;
 constexpr int kRowsWork = 3000;
 
+// Whether a kernel takes the call (its layout, row types, alignments and LDS): asked by the launch and by
+// lf_decode_kernel, which the host's split plan follows.  ``pages``: packed pages of the whole batch.
+bool decode_rows_serves(const DecodeParams& p, int64_t pages);
+bool decode_mfma_serves(const DecodeParams& p);
+bool decode_tiled_serves(const DecodeParams& p);
+
 // Merge the partials of every sequence into ``out`` (enqueued after a decode kernel).  With the
 // host copy of seq_work and at most LF_INLINE_SEQ sequences, the (first, count) pairs go into
 // the reduce kernel's arguments.

@@ -1530,12 +1530,8 @@ bool plan_layout(const lf_packed_layer& L, int g, MfmaLayout& y) {
     return y.lds_bytes <= 160 * 1024 - 64;
 }
 
-}  // namespace
-
-int launch_decode_mfma(const DecodeParams& p, hipStream_t stream, bool* handled) {
-    MfmaParams mp;
-    mp.p = p;
-    mp.k = UnpackBits{0x00C000C0u, 0x03000300u, 0x003C003Cu, 0x03C003C0u, 0x4C004C00u, 0x44004400u, 0x5C005C00u};
+// The call's LDS layout and residual form; false when it is outside this kernel.
+bool serves(const DecodeParams& p, MfmaLayout& y, int& res_mfma) {
     // The residual pass reads 16-byte Key chunks and 4-byte Value pairs of the tail and new rows.
     const bool rows_aligned = (p.A.tail_cap == 0 || (aligned(p.A.tail_k, 16) && aligned(p.A.tail_v, 4))) &&
                               (!p.A.k_new || (aligned(p.A.k_new, 16) && aligned(p.A.v_new, 4)));
@@ -1546,18 +1542,33 @@ int launch_decode_mfma(const DecodeParams& p, hipStream_t stream, bool* handled)
     const bool one_dtype = !has_tail || !has_new || p.A.new_dtype == p.A.tail_dtype;
     const bool rows16 = (!has_tail || (aligned(p.A.tail_k, 16) && aligned(p.A.tail_v, 16))) &&
                         (!has_new || (aligned(p.A.k_new, 16) && aligned(p.A.v_new, 16)));
-    mp.res_mfma = (has_tail || has_new) && one_dtype && rows16 && res_dt != LF_FP32 ? (res_dt == LF_BF16 ? 1 : 2) : 0;
+    res_mfma = (has_tail || has_new) && one_dtype && rows16 && res_dt != LF_FP32 ? (res_dt == LF_BF16 ? 1 : 2) : 0;
     // Several new tokens need the matrix-core residual pass (the VALU pass takes one).
-    const bool res_ok = p.q_len == 1 || mp.res_mfma != 0 || (!has_tail && !has_new);
-    if (!rows_aligned || !res_ok || !plan_layout(p.L, p.g, mp.y)) {
-        *handled = false;
-        return LF_OK;
-    }
+    const bool res_ok = p.q_len == 1 || res_mfma != 0 || (!has_tail && !has_new);
+    return rows_aligned && res_ok && plan_layout(p.L, p.g, y);
+}
+
+}  // namespace
+
+bool decode_mfma_serves(const DecodeParams& p) {
+    MfmaLayout y;
+    int res_mfma;
+    return serves(p, y, res_mfma);
+}
+
+int launch_decode_mfma(const DecodeParams& p, hipStream_t stream, bool* handled) {
+    MfmaParams mp;
+    mp.p = p;
+    mp.k = UnpackBits{0x00C000C0u, 0x03000300u, 0x003C003Cu, 0x03C003C0u, 0x4C004C00u, 0x44004400u, 0x5C005C00u};
+    *handled = serves(p, mp.y, mp.res_mfma);
+    if (!*handled) return LF_OK;
     mp.n_rt = (p.g + 7) / 8;
     const int64_t pairs = static_cast<int64_t>(p.A.n_work) * p.L.n_kv;
     const int64_t blocks = mp.n_rt == 1 ? pairs : (pairs + 7) / 8 * 8 * mp.n_rt;
-    if (blocks > 0x7fffffff) return LF_E_SHAPE;
-    *handled = true;
+    if (blocks > 0x7fffffff) {
+        *handled = false;
+        return LF_E_SHAPE;
+    }
     const int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&decode_mfma_kernel), mp.y.lds_bytes);
     if (rc != LF_OK) return rc;
     const bool grid2d = mp.n_rt == 1 && p.A.n_work <= 65535;

@@ -666,25 +666,33 @@ int launch_rows(const RowsParams& rp, hipStream_t stream) {
     return LF_OK;
 }
 
+bool serves(const DecodeParams& p, int64_t pages, RowsLayout& y) {
+    const int tiles = (p.g + 7) / 8;
+    if (tiles < kRowsTiles || p.A.n_work > 65535 || p.L.n_kv > 65535) return false;
+    if (pages * p.L.n_kv * tiles < kRowsWork) return false;
+    // 2-byte rows of one dtype, read in 16-byte pieces
+    const int dt = p.A.q_dtype;
+    if (dt == LF_FP32 || !aligned(p.A.query, 16)) return false;
+    if (p.A.k_new && (p.A.new_dtype != dt || !aligned(p.A.k_new, 16) || !aligned(p.A.v_new, 16))) return false;
+    if (p.A.tail_cap > 0 && (p.A.tail_dtype != dt || !aligned(p.A.tail_k, 16) || !aligned(p.A.tail_v, 16))) return false;
+    return plan_rows(p.L, y);
+}
+
 }  // namespace
+
+bool decode_rows_serves(const DecodeParams& p, int64_t pages) {
+    RowsLayout y;
+    return serves(p, pages, y);
+}
 
 int launch_decode_rows(const DecodeParams& p, hipStream_t stream, bool* handled) {
     RowsParams rp;
     rp.p = p;
-    *handled = false;
-    const int tiles = (p.g + 7) / 8;
-    if (tiles < kRowsTiles || !p.A.work_host || p.A.n_work > 65535 || p.L.n_kv > 65535) return LF_OK;
     int64_t pages = 0;
-    for (int i = 0; i < p.A.n_work; ++i) pages += p.A.work_host[4 * i + 2] - p.A.work_host[4 * i + 1];
-    if (pages * p.L.n_kv * tiles < kRowsWork) return LF_OK;
-    // 2-byte rows of one dtype, read in 16-byte pieces
-    const int dt = p.A.q_dtype;
-    if (dt == LF_FP32 || !aligned(p.A.query, 16)) return LF_OK;
-    if (p.A.k_new && (p.A.new_dtype != dt || !aligned(p.A.k_new, 16) || !aligned(p.A.v_new, 16))) return LF_OK;
-    if (p.A.tail_cap > 0 && (p.A.tail_dtype != dt || !aligned(p.A.tail_k, 16) || !aligned(p.A.tail_v, 16))) return LF_OK;
-    if (!plan_rows(p.L, rp.y)) return LF_OK;
-    *handled = true;
-    const bool bf = dt == LF_BF16;
+    for (int i = 0; p.A.work_host && i < p.A.n_work; ++i) pages += p.A.work_host[4 * i + 2] - p.A.work_host[4 * i + 1];
+    *handled = serves(p, pages, rp.y);
+    if (!*handled) return LF_OK;
+    const bool bf = p.A.q_dtype == LF_BF16;
     int rc;
     if (p.g > 64) rc = bf ? launch_rows<true, 1>(rp, stream) : launch_rows<false, 1>(rp, stream);
     else rc = bf ? launch_rows<true, 2>(rp, stream) : launch_rows<false, 2>(rp, stream);

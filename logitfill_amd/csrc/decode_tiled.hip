@@ -944,12 +944,21 @@ int launch_tiled_d(const TiledParams& tp, hipStream_t stream) {
     return LF_E_UNSUPPORTED;
 }
 
+bool serves(const DecodeParams& p, TiledLayout& y) {
+    return plan_tiled(p.L, y) && p.A.n_work <= 65535 && (p.g + kRows - 1) / kRows <= 65535;
+}
+
 }  // namespace
+
+bool decode_tiled_serves(const DecodeParams& p) {
+    TiledLayout y;
+    return serves(p, y);
+}
 
 int launch_decode_tiled(const DecodeParams& p, hipStream_t stream, bool* handled) {
     TiledParams tp;
     tp.p = p;
-    *handled = plan_tiled(p.L, tp.y) && p.A.n_work <= 65535 && (p.g + kRows - 1) / kRows <= 65535;
+    *handled = serves(p, tp.y);
     if (!*handled) return LF_OK;
     const bool has_tail = p.A.tail_cap > 0, has_new = p.A.k_new != nullptr;
     tp.res_vec = (!has_tail || (aligned16(p.A.tail_k) && aligned16(p.A.tail_v))) &&

@@ -24,6 +24,7 @@ import functools
 import os
 import warnings
 from collections import Counter
+from typing import NamedTuple
 
 import numpy as np
 import torch
@@ -434,6 +435,67 @@ def kernel_choice() -> int:
     return {"auto": _native.KERNEL_AUTO, "valu": _native.KERNEL_VALU, "mfma": _native.KERNEL_MFMA}[name]
 
 
+# Query rows per workgroup of the matrix-core decode kernels: rows beyond it ((n_q / n_kv) * q_len
+# per kv head) run as further row tiles, each a workgroup of its own over the same pages.
+MFMA_TILE_ROWS = 8
+
+
+class PlanRule(NamedTuple):
+    """How a call's split plan is sized: by the kernel that takes it."""
+    kernel: int            # _native.KERNEL_*
+    tiles: int             # workgroups per (item, kv head): one per tile of query rows
+    page_size: int
+    page_elems: int        # page_size x head_dim
+    per_cu: int            # workgroups a CU holds
+    one_round: bool        # sizes above the even share where only they make one round
+    dispatch_order: bool   # paired_split and age_split (decode_mfma.hip's dispatch order, one row tile)
+
+    def residual(self, tail: int, q_len: int) -> int:
+        """Cost of the residual (longest tail and ``q_len`` new tokens) in packed pages."""
+        P = self.page_size
+        if self.kernel == _native.KERNEL_ROWS:
+            # a dense chunk of 128 tail and new tokens costs about a page there
+            return 1 + -(-(tail + q_len) // P)
+        # q_len new tokens lengthen the residual (a chunk of 128 tokens more past a full page)
+        pages = residual_pages((tail,)) + (tail + q_len - 1) // P * (RESIDUAL_FIXED_PAGES + RESIDUAL_TAIL_PAGES)
+        return pages if self.page_elems == 128 * 128 else scaled_pages(pages, self.page_elems)
+
+
+def _tail_args(a, tail_k, tail_v) -> None:
+    if tail_k is not None:
+        a.tail_k = tail_k.data_ptr()
+        a.tail_v = tail_v.data_ptr()
+        a.tail_dtype = _native.dtype_code(tail_k.dtype)
+        a.tail_cap = int(tail_k.shape[2])
+    else:
+        a.tail_dtype = _native.LF_BF16
+        a.tail_cap = 0
+
+
+def plan_rule(manager, layer, call: tuple, q_ptr: int, k_ptr: int, v_ptr: int) -> PlanRule:
+    """The rule for ``call`` (history pages, q_len, kernel, row dtypes ...; see ``decode_into``), from the
+    library's own choice of kernel.  A call the library refuses gets decode_mfma.hip's; the launch
+    reports it."""
+    hist_pages, q_len, kernel, q_dtype, new_dtype = call[:5]
+    a = _native.DecodeArgs()
+    a.query, a.k_new, a.v_new = q_ptr, k_ptr, v_ptr
+    a.q_dtype = a.out_dtype = _native.dtype_code(q_dtype)
+    if new_dtype is not None:
+        a.new_dtype = _native.dtype_code(new_dtype)
+    _tail_args(a, *layer.tail_buffers())
+    a.n_q, a.q_len, a.kernel = manager.n_q, q_len, kernel
+    taken = _native.load().lf_decode_kernel(layer.layer_struct(), a, sum(hist_pages))
+    if taken < 0:
+        taken = _native.KERNEL_MFMA
+    rows = manager.n_q // manager.n_kv * q_len
+    mfma = taken == _native.KERNEL_MFMA
+    wide = taken == _native.KERNEL_ROWS  # 64 or 128 rows a workgroup, which fills a CU
+    tiles = -(-rows // ((128 if rows > 64 else 64) if wide else MFMA_TILE_ROWS))
+    # (the other kernels gain and lose by one-round sizes: 0.75 to 1.33 times, 26 layouts and batches)
+    return PlanRule(taken, tiles, layer.page_size, layer.page_size * layer.head_dim, 1 if wide else 2, mfma or wide,
+                    mfma and tiles == 1)
+
+
 def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new, scaling: float,
                 out: torch.Tensor, kernel: int | None = None, pages_per_split: int | None = None,
                 noalloc: bool = False, commit: bool = False) -> bool:
@@ -468,37 +530,31 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
     kernel = kernel_choice() if kernel is None else kernel
     P = layer.page_size
     hist_pages = tuple(h // P for h in layer.hist_lens)
-    # q_len new tokens lengthen the residual (a chunk of 128 tokens more past a full page)
-    res_pages = residual_pages(layer.tail_lens) + (max(layer.tail_lens, default=0) + q_len - 1) // P * (
-        RESIDUAL_FIXED_PAGES + RESIDUAL_TAIL_PAGES)
-    page_elems = P * D
-    if page_elems != 128 * 128:
-        res_pages = scaled_pages(res_pages, page_elems)
-    # workgroups per (item, kv head): one per tile of query rows
-    rows = manager.n_q // manager.n_kv * q_len
-    default_layout = P == layer.k_group_size == layer.v_group_size == D == 128
-    # decode_mfma.hip takes the call (fp32 rows of several tokens go to decode_tiled.hip); the other
-    # kernels gain and lose by one-round sizes (0.75 to 1.33 times, 26 layouts and batches)
-    one_round = default_layout and kernel != _native.KERNEL_VALU and (q_len == 1 or query.dtype != torch.float32)
-    tiles = -(-rows // MFMA_TILE_ROWS)
-    # decode_rows.hip takes the call
-    wide = (tiles >= ROWS_TILES and sum(hist_pages) * layer.n_kv * tiles >= ROWS_WORK and default_layout
-            and kernel == _native.KERNEL_AUTO and query.dtype != torch.float32)
-    if wide:
-        tiles = -(-rows // rows_tile(rows))
-        # a dense chunk of 128 tail and new tokens costs about a page there
-        res_pages = 1 + -(-(max(layer.tail_lens, default=0) + q_len) // P)
+    tail_k, tail_v = layer.tail_buffers()
+    if key_new is not None and value_new.dtype != key_new.dtype:
+        raise TypeError("key_new and value_new must share a dtype")
+    q_ptr, k_ptr, v_ptr = query.data_ptr(), 0, 0
+    if key_new is not None:
+        k_ptr, v_ptr = key_new.data_ptr(), value_new.data_ptr()
+    # which kernel takes the call, and so how its plan is sized: asked again when something it
+    # depends on changes
+    rule_key = (hist_pages, q_len, kernel, query.dtype, None if key_new is None else key_new.dtype,
+                None if tail_k is None else tail_k.dtype, (q_ptr & 15) << 8 | (k_ptr & 15) << 4 | v_ptr & 15)
+    cached_rule = layer.__dict__.get("_lf_plan_rule")
+    if cached_rule is None or cached_rule[0] != rule_key:
+        cached_rule = (rule_key, plan_rule(manager, layer, rule_key, q_ptr, k_ptr, v_ptr))
+        layer.__dict__["_lf_plan_rule"] = cached_rule
+    rule = cached_rule[1]
+    res_pages = rule.residual(max(layer.tail_lens), q_len)
     if pages_per_split is None:
-        # the split depends on the history, the residual cost, the environment's override and
-        # whether the dispatch order of decode_mfma.hip applies (its layout, one row tile): chosen
-        # again when one changes
-        age = kernel != _native.KERNEL_VALU and tiles == 1 and not wide and default_layout
-        choice_key = (hist_pages, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"), age, tiles, wide, one_round)
+        # the split depends on the history, the kernel, the residual cost and the environment's
+        # override: chosen again when one changes
+        choice_key = (hist_pages, rule, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"))
         cached = layer.__dict__.get("_lf_split_choice")
         if cached is None or cached[0] != choice_key:
-            size = choose_pages_per_split(list(hist_pages), layer.n_kv * tiles, res_pages, layer.device, page_elems,
-                                          1 if wide else 2, one_round)
-            if age and choice_key[2] is None:
+            size = choose_pages_per_split(list(hist_pages), layer.n_kv * rule.tiles, res_pages, layer.device,
+                                          rule.page_elems, rule.per_cu, rule.one_round)
+            if rule.dispatch_order and choice_key[3] is None:
                 cus = _cu_count(layer.device)
                 paired = paired_split(list(hist_pages), layer.n_kv, res_pages, cus, size)
                 if paired is not None:
@@ -529,9 +585,6 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
         ws_need = (wkey, lib.lf_decode_workspace_bytes(wkey[0], wkey[1], plan.n_work))
         plan.__dict__["_lf_ws_bytes"] = ws_need
     ws = None if noalloc else manager.workspace(ws_need[1])
-    tail_k, tail_v = layer.tail_buffers()
-    if key_new is not None and value_new.dtype != key_new.dtype:
-        raise TypeError("key_new and value_new must share a dtype")
     tail_len = layer.tail_len_device()
     # Every field but the four per-call tensors is fixed while the plan, the buffers and the
     # call's settings stay the same: the argument block is kept on the layer and reused.  The
@@ -548,14 +601,7 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
         a.q_dtype = _native.dtype_code(query.dtype)
         if key_new is not None:
             a.new_dtype = _native.dtype_code(key_new.dtype)
-        if tail_k is not None:
-            a.tail_k = tail_k.data_ptr()
-            a.tail_v = tail_v.data_ptr()
-            a.tail_dtype = _native.dtype_code(tail_k.dtype)
-            a.tail_cap = int(tail_k.shape[2])
-        else:
-            a.tail_dtype = _native.LF_BF16
-            a.tail_cap = 0
+        _tail_args(a, tail_k, tail_v)
         a.tail_len = tail_len.data_ptr()
         a.out_dtype = _native.dtype_code(out.dtype)
         a.n_q = manager.n_q
@@ -570,10 +616,10 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
         a.kernel = kernel
         a.q_len = q_len
         layer.__dict__["_lf_decode_args"] = (static_key, a, held)
-    a.query = query.data_ptr()
+    a.query = q_ptr
     a.out = out.data_ptr()
-    a.k_new = 0 if key_new is None else key_new.data_ptr()
-    a.v_new = 0 if key_new is None else value_new.data_ptr()
+    a.k_new = k_ptr
+    a.v_new = v_ptr
     # the commit folds into the launch while every sequence's residual page stays below full
     fold = commit and key_new is not None and tail_k is not None and max(layer.tail_lens) + q_len < P
     a.commit_new = 1 if fold else 0
@@ -602,21 +648,6 @@ def _kernel_attention(manager, layer_idx: int, query: torch.Tensor, key_new: tor
     out = torch.empty(B, n_q, q_len, D, dtype=query.dtype, device=query.device)
     folded = decode_into(manager, layer_idx, q, kn, vn, scaling, out, commit=commit)
     return out, folded
-
-
-# Query rows per workgroup of the matrix-core decode kernel: rows beyond it ((n_q / n_kv) * q_len
-# per kv head) run as further row tiles, each a workgroup of its own over the same pages.
-MFMA_TILE_ROWS = 8
-
-# Calls of at least this many tiles of MFMA_TILE_ROWS rows and this many page-tiles (pages x kv heads
-# x tiles) run decode_rows.hip (kRowsTiles, kRowsWork there, with the measurements).
-ROWS_TILES = 6
-ROWS_WORK = 3000
-
-
-def rows_tile(rows: int) -> int:
-    """Query rows per workgroup of decode_rows.hip for ``rows`` rows per kv head."""
-    return 128 if rows > 64 else 64
 
 
 def valu_tile_rows(head_dim: int) -> int:
