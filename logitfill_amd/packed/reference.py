@@ -160,7 +160,8 @@ def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
 
 
 def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int, device=None,
-                           page_elems: int = 128 * 128, per_cu: int = 2, one_round: bool = False) -> int:
+                           page_elems: int = 128 * 128, per_cu: int = 2, one_round: bool = False,
+                           overhead: int | None = None) -> int:
     """Work per split-K item, in pages.  The decode kernel holds two workgroups per CU (the
     slots).  Items of ``total work / slots`` pages fill the slots once when every sequence's
     work (its pages plus its residual) divides evenly; with ragged lengths the per-sequence
@@ -175,13 +176,15 @@ def choose_pages_per_split(hist_pages: list[int], n_kv: int, residual_pages: int
     pages of head_dim 64 (8 sequences of 50 pages, 2 kv heads) take 4-page items, 15.0 us per
     layer-step, instead of the 2-page ones of an unscaled cost, 18.2.  ``per_cu``: workgroups a
     CU holds (one of decode_rows.hip).  ``one_round``: sizes above the even share may make the
-    one round that no smaller size does."""
+    one round that no smaller size does.  ``overhead``: the per-item cost in pages of this layout, where
+    it is not that of ``ITEM_OVERHEAD_PAGES``."""
     forced = env_int("LOGITFILL_AMD_PAGES_PER_SPLIT", 0)
     if forced > 0:
         return forced
     slots = per_cu * (_cu_count(device) if device is not None else 256)
     return _pages_per_split(tuple(int(x) for x in hist_pages), int(n_kv), int(residual_pages), slots,
-                            scaled_pages(ITEM_OVERHEAD_PAGES, page_elems), per_cu, bool(one_round))
+                            scaled_pages(ITEM_OVERHEAD_PAGES, page_elems) if overhead is None else overhead, per_cu,
+                            bool(one_round))
 
 
 # Of the two decode workgroups that share a CU, the one dispatched second runs this much slower
@@ -440,6 +443,18 @@ def kernel_choice() -> int:
 MFMA_TILE_ROWS = 8
 
 
+# decode_valu.hip: one wave per workgroup, whose time is its pages' (27 us a 128-token page at head_dim
+# 32, 110 at 128) on 30 us of fixed cost, four to a CU or more where its LDS allows.  Items of one page
+# up to four workgroups per CU (us a call: the plan this kernel had under decode_mfma.hip's costs / with
+# those costs scaled to the page / this one): head_dim 32, 8 sequences of 1.5K-5K tokens 108 / 253 / 109;
+# head_dim 16, 64-token pages 94 / 180 / 43 and, 3 tokens, 159 / 596 / 69; 16-token pages of head_dim 128
+# 416 / 859 / 251; Value groups of 8 697 / 1 122 / 467; head_dim 512 1 468 / 2 293 / 1 419, with 64-token
+# pages 682 / 716 / 715.  Over 19 layouts x 1 and 3 tokens 0.95 to 6.5 times the first, 1.0 to 16 times the
+# second.
+GENERAL_PER_CU = 4
+GENERAL_OVERHEAD = 1
+
+
 class PlanRule(NamedTuple):
     """How a call's split plan is sized: by the kernel that takes it."""
     kernel: int            # _native.KERNEL_*
@@ -447,6 +462,7 @@ class PlanRule(NamedTuple):
     page_size: int
     page_elems: int        # page_size x head_dim
     per_cu: int            # workgroups a CU holds
+    overhead: int | None   # an item's fixed cost in pages (None: ITEM_OVERHEAD_PAGES of 128 x 128)
     one_round: bool        # sizes above the even share where only they make one round
     dispatch_order: bool   # paired_split and age_split (decode_mfma.hip's dispatch order, one row tile)
 
@@ -456,6 +472,8 @@ class PlanRule(NamedTuple):
         if self.kernel == _native.KERNEL_ROWS:
             # a dense chunk of 128 tail and new tokens costs about a page there
             return 1 + -(-(tail + q_len) // P)
+        if self.kernel == _native.KERNEL_VALU:
+            return 1 + (tail + q_len - 1) // P
         # q_len new tokens lengthen the residual (a chunk of 128 tokens more past a full page)
         pages = residual_pages((tail,)) + (tail + q_len - 1) // P * (RESIDUAL_FIXED_PAGES + RESIDUAL_TAIL_PAGES)
         return pages if self.page_elems == 128 * 128 else scaled_pages(pages, self.page_elems)
@@ -490,10 +508,23 @@ def plan_rule(manager, layer, call: tuple, q_ptr: int, k_ptr: int, v_ptr: int) -
     rows = manager.n_q // manager.n_kv * q_len
     mfma = taken == _native.KERNEL_MFMA
     wide = taken == _native.KERNEL_ROWS  # 64 or 128 rows a workgroup, which fills a CU
-    tiles = -(-rows // ((128 if rows > 64 else 64) if wide else MFMA_TILE_ROWS))
+    general = taken == _native.KERNEL_VALU
+    tile = valu_tile_rows(layer.head_dim) if general else (128 if rows > 64 else 64) if wide else MFMA_TILE_ROWS
+    tiles = -(-rows // tile)
     # (the other kernels gain and lose by one-round sizes: 0.75 to 1.33 times, 26 layouts and batches)
-    return PlanRule(taken, tiles, layer.page_size, layer.page_size * layer.head_dim, 1 if wide else 2, mfma or wide,
-                    mfma and tiles == 1)
+    return PlanRule(taken, tiles, layer.page_size, layer.page_size * layer.head_dim,
+                    GENERAL_PER_CU if general else 1 if wide else 2, GENERAL_OVERHEAD if general else None,
+                    mfma or wide, mfma and tiles == 1)
+
+
+def fit_scratch(size: int, hist_pages, residual: int, item_bytes: int) -> int:
+    """``size`` doubled until the items' partials fit the scratch array of the call that allocates nothing
+    (or every sequence is one item)."""
+    limit = _native.load().lf_noalloc_scratch_bytes()
+    while size < max(hist_pages) + residual and item_bytes * sum(
+            1 if p == 0 else -(-(p + residual) // size) for p in hist_pages) > limit:
+        size *= 2
+    return size
 
 
 def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new, scaling: float,
@@ -528,6 +559,7 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
             _expect(key_new, want_kv, "key_new")
             _expect(value_new, want_kv, "value_new")
     kernel = kernel_choice() if kernel is None else kernel
+    lib = _native.load()
     P = layer.page_size
     hist_pages = tuple(h // P for h in layer.hist_lens)
     tail_k, tail_v = layer.tail_buffers()
@@ -549,11 +581,13 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
     if pages_per_split is None:
         # the split depends on the history, the kernel, the residual cost and the environment's
         # override: chosen again when one changes
-        choice_key = (hist_pages, rule, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"))
+        choice_key = (hist_pages, rule, res_pages, os.environ.get("LOGITFILL_AMD_PAGES_PER_SPLIT"), noalloc)
         cached = layer.__dict__.get("_lf_split_choice")
         if cached is None or cached[0] != choice_key:
             size = choose_pages_per_split(list(hist_pages), layer.n_kv * rule.tiles, res_pages, layer.device,
-                                          rule.page_elems, rule.per_cu, rule.one_round)
+                                          rule.page_elems, rule.per_cu, rule.one_round, rule.overhead)
+            if noalloc and rule.kernel == _native.KERNEL_VALU and choice_key[3] is None:
+                size = fit_scratch(size, hist_pages, res_pages, lib.lf_decode_workspace_bytes(manager.n_q * q_len, D, 1))
             if rule.dispatch_order and choice_key[3] is None:
                 cus = _cu_count(layer.device)
                 paired = paired_split(list(hist_pages), layer.n_kv, res_pages, cus, size)
@@ -578,7 +612,6 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
             plan = DecodePlan(list(hist_pages), layer.n_kv, pages_per_split, layer.device, res_pages)
             shared[pkey] = plan
         layer.decode_plan = plan
-    lib = _native.load()
     wkey = (manager.n_q * q_len, layer.head_dim)
     ws_need = plan.__dict__.get("_lf_ws_bytes")
     if ws_need is None or ws_need[0] != wkey:

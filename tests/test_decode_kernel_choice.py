@@ -9,7 +9,7 @@ import torch
 
 from logitfill_amd import _native
 from logitfill_amd.packed.layout import sm_page_elems
-from logitfill_amd.packed.reference import plan_rule
+from logitfill_amd.packed.reference import choose_pages_per_split, fit_scratch, plan_rule
 
 VALU, MFMA, ROWS, TILED = (_native.KERNEL_VALU, _native.KERNEL_MFMA, _native.KERNEL_ROWS, _native.KERNEL_TILED)
 AT = 1 << 20  # an address (nothing reads it)
@@ -101,3 +101,31 @@ def test_plan_follows_the_kernel():
     assert rule.kernel == TILED and rule.per_cu == 2 and not rule.one_round and not rule.dispatch_order
     assert _rule(8, 1, bf, bf, bf, 500, kg=32).kernel == TILED
     assert _rule(8, 1, bf, bf, bf, 500, kg=32, kernel=2).kernel == MFMA  # refused by the launch
+
+
+@pytest.mark.parametrize("pages,n_q,q_len,layer,want", [
+    # head_dim 32, 16-row tiles: two kv heads' worth of the work below runs as one-page items
+    ([39, 25, 21, 34, 25, 20, 36, 24], 7, 1, {"D": 32, "vg": 32, "widths": (20, 6, 4, 2)}, 1),
+    ([39, 25, 21, 34, 25, 20, 36, 24], 7, 3, {"D": 32, "vg": 32, "widths": (20, 6, 4, 2)}, 1),
+    ([62, 35, 28, 53, 36, 25, 56, 32], 4, 1, {"D": 16, "page": 64, "kg": 64, "vg": 16, "widths": (10, 3, 2, 1)}, 1),
+    ([187, 109, 173, 63], 7, 1, {"page": 16, "kg": 16, "vg": 32}, 1),
+    ([600] * 8, 7, 1, {"page": 16, "kg": 16, "vg": 32}, 5),            # 4 800 pages: 1 024 slots once
+])
+def test_general_kernel_items_stay_small(pages, n_q, q_len, layer, want):
+    """The general kernel's plan: small items, up to four workgroups per CU (with the matrix-core
+    kernels' per-item cost it took items of 3 to 16 pages here, up to four times slower)."""
+    bf = torch.bfloat16
+    rule = _rule(n_q, q_len, bf, bf, bf, sum(pages), **layer)
+    assert rule.kernel == VALU and rule.tiles == -(-n_q * q_len // 16)
+    res = rule.residual(50 % rule.page_size, q_len)
+    assert res == 1
+    assert choose_pages_per_split(pages, rule.tiles, res, None, rule.page_elems, rule.per_cu, rule.one_round,
+                                  rule.overhead) == want
+
+
+def test_plan_of_a_call_that_allocates_nothing_fits_its_scratch():
+    limit = _native.load().lf_noalloc_scratch_bytes()
+    assert fit_scratch(1, [100] * 8, 1, limit // 1000) == 1
+    assert fit_scratch(1, [100] * 8, 1, limit // 500) == 2
+    assert fit_scratch(3, [100, 0, 40], 1, limit // 10) == 24           # 5 + 1 + 2 items
+    assert fit_scratch(1, [100] * 8, 1, limit) >= 101                    # cannot fit: one item a sequence
