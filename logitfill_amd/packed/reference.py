@@ -133,6 +133,16 @@ ITEM_OVERHEAD_PAGES = 5
 ALONE_FACTOR = 0.78
 
 
+# A size past the even share that makes one round is taken where its estimate is this much better than
+# the smaller items' rounds, and for one, two or four row tiles.  2 800 drawn batches with such a size: 0.96
+# to 1.55 times the speed of the smaller items, median 1.16, two below 0.98.  At an estimated gain below
+# 1.02 the median is 1.00 (140 batches, from 0.94).  Three and five tiles do not divide the 64 slots of an
+# XCD, which the tiles of an (item, kv head) share (decode_mfma.hip): 760 batches 0.63 to 1.5 times, median
+# 0.83 where an XCD gets a 65th workgroup.
+ONE_ROUND_GAIN = 1.07
+ONE_ROUND_TILES = (1, 2, 4)
+
+
 @functools.lru_cache(maxsize=256)
 def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
                      overhead: int = ITEM_OVERHEAD_PAGES, per_cu: int = 2, one_round: bool = False) -> int:
@@ -143,7 +153,7 @@ def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
     # itself, or when it is what makes one round of ragged sequences whose rounded-up items overflow
     # the slots at the even share (us per layer-step, two rounds / one: 669 pages in 16 sequences, 4 kv
     # heads, 4 row tiles, 15- / 34-page items 67.3 / 61.8, 2 tiles, 7 / 15 pages 45.0 / 37.0; 840 in 12, 8
-    # kv heads, 1 tile, 8 / 18 pages 48.0 / 39.6; 40 drawn batches 1.00 to 1.32 times, one 0.98).
+    # kv heads, 1 tile, 8 / 18 pages 48.0 / 39.6).  The estimate has to be ONE_ROUND_GAIN better.
     size = np.arange(max(top, int(work.max())), 0, -1, dtype=np.int64)[:, None]   # largest first
     items = np.where(p[None, :] == 0, 1, -(-work[None, :] // size))   # lf_plan_decode's count
     wgs = n_kv * items.sum(axis=1)
@@ -155,7 +165,8 @@ def _pages_per_split(pages: tuple, n_kv: int, residual_pages: int, slots: int,
     if per_cu == 2:
         fits = rounds == 1
         past = size[:, 0] > top
-        cost = np.where(past & ~alone & ~(one_round & fits & ~np.any(fits & ~past)), np.inf, cost)
+        better = cost * ONE_ROUND_GAIN <= cost[~past].min()
+        cost = np.where(past & ~alone & ~(one_round & fits & better & ~np.any(fits & ~past)), np.inf, cost)
     return int(size[int(np.argmin(cost)), 0])                          # ties: fewest items
 
 
@@ -514,7 +525,7 @@ def plan_rule(manager, layer, call: tuple, q_ptr: int, k_ptr: int, v_ptr: int) -
     # (the other kernels gain and lose by one-round sizes: 0.75 to 1.33 times, 26 layouts and batches)
     return PlanRule(taken, tiles, layer.page_size, layer.page_size * layer.head_dim,
                     GENERAL_PER_CU if general else 1 if wide else 2, GENERAL_OVERHEAD if general else None,
-                    mfma or wide, mfma and tiles == 1)
+                    mfma and tiles in ONE_ROUND_TILES, mfma and tiles == 1)
 
 
 def fit_scratch(size: int, hist_pages, residual: int, item_bytes: int) -> int:

@@ -94,9 +94,12 @@ def test_plan_follows_the_kernel():
     for other in (_rule(48, 1, bf, bf, fp16, 500), _rule(48, 1, bf, bf, bf, 500, q_at=AT + 2),
                   _rule(48, 1, fp32, fp32, fp32, 500), _rule(48, 1, bf, bf, bf, 400),
                   _rule(48, 1, bf, bf, bf, 500, widths=(30, 4, 4, 90))):
-        assert other.kernel == MFMA and other.per_cu == 2 and other.tiles == 6 and other.one_round
+        assert other.kernel == MFMA and other.per_cu == 2 and other.tiles == 6 and not other.one_round
     rule = _rule(8, 1, bf, bf, bf, 500)
     assert rule.kernel == MFMA and rule.dispatch_order and rule.residual(100, 1) == 4
+    for n_q, tiles in ((8, 1), (16, 2), (20, 3), (32, 4), (36, 5)):
+        rule = _rule(n_q, 1, bf, bf, bf, 100)
+        assert rule.tiles == tiles and rule.one_round == (tiles in (1, 2, 4))
     rule = _rule(8, 6, bf, bf, fp32, 500)     # rows of two types, several tokens
     assert rule.kernel == TILED and rule.per_cu == 2 and not rule.one_round and not rule.dispatch_order
     assert _rule(8, 1, bf, bf, bf, 500, kg=32).kernel == TILED

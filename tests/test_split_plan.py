@@ -302,3 +302,29 @@ def test_one_round_size(pages, n_kv, res, slots=512):
     for b, p0, p1, _ in plan_items(pages, size, res):
         covered[b] += p1 - p0
     assert covered == list(pages)
+
+
+def test_one_round_size_needs_a_clear_gain(slots=512):
+    """A size past the even share is taken only where its estimate (largest item + overhead, one round)
+    beats the smaller sizes' by 7 %; drawn batches of both kinds occur."""
+    rng = np.random.default_rng(3)
+    taken = declined = 0
+    for _ in range(1500):
+        n_kv = int(rng.choice([2, 4, 8]))
+        pages = [int(x) for x in rng.integers(1, 300, int(rng.integers(2, 33)))]
+        even = max(1, -(-n_kv * (sum(pages) + 4 * len(pages)) // slots))
+        before = choose_pages_per_split(pages, n_kv, 4)
+        size = choose_pages_per_split(pages, n_kv, 4, one_round=True)
+        if size <= even or size == before:
+            declined += 1
+            assert size == before
+            continue
+
+        def cost(s):
+            items = [-(-(p + 4) // s) for p in pages]
+            rounds = -(-n_kv * sum(items) // slots)
+            return rounds * (max(-(-(p + 4) // k) for p, k in zip(pages, items)) + ITEM_OVERHEAD_PAGES), rounds
+
+        taken += 1
+        assert cost(size)[1] == 1 and 1.07 * cost(size)[0] <= min(cost(s)[0] for s in range(1, even + 1))
+    assert taken > 50 and declined > 50
