@@ -124,6 +124,16 @@ int32_t lf_pack_pages(const lf_packed_layer* layer,
                       int64_t src_stride_b, int64_t src_stride_h, int64_t src_stride_t,
                       const int32_t* jobs, int32_t n_jobs, void* stream);
 
+/*
+ * The kernel lf_pack_pages takes for this layer and source (host function, no device access; nothing is
+ * read through the pointers): an LF_PACK_* value or a negative LF_E_*.
+ */
+#define LF_PACK_GENERAL 1
+#define LF_PACK_FAST 2   /* 128-channel heads, 128-token pages and groups, int2 Values */
+#define LF_PACK_TILED 3  /* the other layouts of aligned 2-byte rows */
+int32_t lf_pack_kernel(const lf_packed_layer* layer, const void* k_src, const void* v_src, int32_t src_dtype,
+                       int64_t src_stride_b, int64_t src_stride_h, int64_t src_stride_t);
+
 /* Page source of one layer for lf_pack_pages_multi: element strides, channel stride 1. */
 typedef struct lf_pack_source {
     const void* k;

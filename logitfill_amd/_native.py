@@ -18,6 +18,8 @@ LF_OK, LF_E_NULL, LF_E_SHAPE, LF_E_UNSUPPORTED, LF_E_WORKSPACE, LF_E_DTYPE = 0, 
 KERNEL_AUTO, KERNEL_VALU, KERNEL_MFMA = 0, 1, 2
 # the kernels a call can take (lf_decode_kernel)
 KERNEL_ROWS, KERNEL_TILED = 3, 4
+# the page packers (lf_pack_kernel)
+PACK_GENERAL, PACK_FAST, PACK_TILED = 1, 2, 3
 
 
 class NativeLibraryMissing(RuntimeError):
@@ -99,6 +101,7 @@ _SIGNATURES = {
     "lf_status_string": (c_char_p, [c_int32]),
     "lf_pack_pages": (c_int32, [POINTER(PackedLayer), c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int64,
                                 c_void_p, c_int32, c_void_p]),
+    "lf_pack_kernel": (c_int32, [POINTER(PackedLayer), c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int64]),
     "lf_pack_pages_multi": (c_int32, [c_void_p, POINTER(PackedLayer), c_void_p, POINTER(PackSource), c_int32,
                                       c_int32, c_void_p, c_int32, c_void_p]),
     "lf_plan_decode": (c_int32, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_int32, c_void_p]),

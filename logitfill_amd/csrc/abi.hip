@@ -11,6 +11,8 @@ int launch_pack_pages(const lf_packed_layer& L, const void* k_src, const void* v
 int launch_pack_pages_multi(const lf_packed_layer* layers_dev, const lf_packed_layer* layers_host,
                             const lf_pack_source* srcs_dev, const lf_pack_source* srcs_host, int n_layers,
                             int src_dtype, const int32_t* jobs, int n_jobs, hipStream_t stream);
+int pack_kernel(const lf_packed_layer& L, const void* k_src, const void* v_src, int src_dtype, int64_t sb, int64_t sh,
+                int64_t st);
 int launch_decode_valu(const DecodeParams& p, hipStream_t stream);
 int launch_decode_mfma(const DecodeParams& p, hipStream_t stream, bool* handled);
 int launch_decode_rows(const DecodeParams& p, hipStream_t stream, bool* handled);
@@ -181,6 +183,15 @@ int32_t lf_pack_pages(const lf_packed_layer* layer, const void* k_src, const voi
     if (layer->page_size > 1024 || layer->head_dim > 1024) return LF_E_SHAPE;
     return lf::launch_pack_pages(*layer, k_src, v_src, src_dtype, src_stride_b, src_stride_h, src_stride_t,
                                  jobs, n_jobs, static_cast<hipStream_t>(stream));
+}
+
+int32_t lf_pack_kernel(const lf_packed_layer* layer, const void* k_src, const void* v_src, int32_t src_dtype,
+                       int64_t src_stride_b, int64_t src_stride_h, int64_t src_stride_t) {
+    const int32_t st = check_layer(layer);
+    if (st != LF_OK) return st;
+    if (!valid_dtype(src_dtype)) return LF_E_DTYPE;
+    if (layer->page_size > 1024 || layer->head_dim > 1024) return LF_E_SHAPE;
+    return lf::pack_kernel(*layer, k_src, v_src, src_dtype, src_stride_b, src_stride_h, src_stride_t);
 }
 
 int32_t lf_pack_pages_multi(const lf_packed_layer* layers_dev, const lf_packed_layer* layers_host,

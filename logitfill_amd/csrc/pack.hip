@@ -1207,6 +1207,22 @@ int launch_one(const PackJobArgs& a, dim3 grid, int elem, hipStream_t stream) {
 
 }  // namespace
 
+// Every page row of the source starts on 16 bytes.
+static bool rows_aligned16(const void* k_src, const void* v_src, int src_dtype, int64_t sb, int64_t sh, int64_t st) {
+    const int elem = src_dtype == LF_FP32 ? 4 : 2;
+    const uintptr_t kp = reinterpret_cast<uintptr_t>(k_src), vp = reinterpret_cast<uintptr_t>(v_src);
+    return ((kp | vp) % 16 == 0) && ((sb * elem) % 16 == 0) && ((sh * elem) % 16 == 0) && ((st * elem) % 16 == 0);
+}
+
+int pack_kernel(const lf_packed_layer& L, const void* k_src, const void* v_src, int src_dtype, int64_t sb, int64_t sh,
+                int64_t st) {
+    const bool vec16 = rows_aligned16(k_src, v_src, src_dtype, sb, sh, st);
+    if (pack_fast_ok(L, src_dtype, vec16, st)) return LF_PACK_FAST;
+    const int tb = pack_tile_tokens(L, src_dtype, vec16);
+    if (tb != 0 && tile_lds(L, tb).total <= 160 * 1024 && 2 * (L.page_size / tb) <= 65535) return LF_PACK_TILED;
+    return LF_PACK_GENERAL;
+}
+
 int launch_pack_pages(const lf_packed_layer& L, const void* k_src, const void* v_src, int src_dtype,
                       int64_t sb, int64_t sh, int64_t st, const int32_t* jobs, int n_jobs,
                       hipStream_t stream) {
@@ -1219,12 +1235,11 @@ int launch_pack_pages(const lf_packed_layer& L, const void* k_src, const void* v
     a.st = st;
     a.jobs = jobs;
     const int elem = src_dtype == LF_FP32 ? 4 : 2;
-    const uintptr_t kp = reinterpret_cast<uintptr_t>(k_src), vp = reinterpret_cast<uintptr_t>(v_src);
-    a.vec16 = ((kp | vp) % 16 == 0) && ((sb * elem) % 16 == 0) && ((sh * elem) % 16 == 0) &&
-              ((st * elem) % 16 == 0);
+    a.vec16 = rows_aligned16(k_src, v_src, src_dtype, sb, sh, st);
     a.cw = pack_code_row(L);
     dim3 grid(n_jobs, L.n_kv);
-    if (pack_fast_ok(L, src_dtype, a.vec16 != 0, st)) {
+    const int kernel = pack_kernel(L, k_src, v_src, src_dtype, sb, sh, st);
+    if (kernel == LF_PACK_FAST) {
         const int ld = code_ld(L);
         const size_t lds = pack_fast_lds_bytes(ld, L.k_width[3]);
         const bool half = src_dtype == LF_FP16;
@@ -1232,13 +1247,12 @@ int launch_pack_pages(const lf_packed_layer& L, const void* k_src, const void* v
         return ld == kCodeLdNarrow ? launch_fast_single<kCodeLdNarrow>(a, half, grid2, lds, stream)
                                    : launch_fast_single<kCodeLdWide>(a, half, grid2, lds, stream);
     }
-    if (const int tb = pack_tile_tokens(L, src_dtype, a.vec16 != 0)) {
+    if (kernel == LF_PACK_TILED) {
+        const int tb = pack_tile_tokens(L, src_dtype, a.vec16 != 0);
         const size_t lds = static_cast<size_t>(tile_lds(L, tb).total);
-        if (lds <= 160 * 1024 && 2 * (L.page_size / tb) <= 65535) {
-            const PackTileArgs ta{a, tb};
-            const dim3 tiles(n_jobs, L.n_kv, 2 * (L.page_size / tb));  // z: block of the page, Key and Value
-            return src_dtype == LF_FP16 ? launch_tile<true>(ta, tiles, lds, stream) : launch_tile<false>(ta, tiles, lds, stream);
-        }
+        const PackTileArgs ta{a, tb};
+        const dim3 tiles(n_jobs, L.n_kv, 2 * (L.page_size / tb));  // z: block of the page, Key and Value
+        return src_dtype == LF_FP16 ? launch_tile<true>(ta, tiles, lds, stream) : launch_tile<false>(ta, tiles, lds, stream);
     }
     int rc;
     if (src_dtype == LF_BF16) rc = launch_one<uint16_t, false>(a, grid, elem, stream);

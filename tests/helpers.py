@@ -5,6 +5,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from logitfill_amd import _native
 from oracle import attention as oatt
 from oracle import history as ohist
 
@@ -49,6 +50,19 @@ def assert_history_equal(layer, b, store, *, tail=True):
             tk, tv = layer.tail_buffers()
             assert np.array_equal(f32(tk[b, :, :tl]), store.tail_k)
             assert np.array_equal(f32(tv[b, :, :tl]), store.tail_v)
+
+
+def decode_kernel(mgr, layer: int = 0) -> int:
+    """The kernel (_native.KERNEL_*) that the layer's last attention call took: the library's answer for
+    that call (lf_decode_kernel), which its launch goes by too."""
+    return mgr.layers[layer].__dict__["_lf_plan_rule"][1].kernel
+
+
+def pack_kernel(mgr, key: torch.Tensor, value: torch.Tensor, layer: int = 0) -> int:
+    """The kernel (_native.PACK_*) that packs pages of ``key / value`` [B, n_kv, T, D]."""
+    assert key.stride() == value.stride()
+    return _native.load().lf_pack_kernel(mgr.layers[layer].layer_struct(), key.data_ptr(), value.data_ptr(),
+                                         _native.dtype_code(key.dtype), *key.stride()[:3])
 
 
 def ulp(x: np.ndarray, dtype: str) -> np.ndarray:

@@ -9,6 +9,7 @@ import torch
 from logitfill_amd import _native, synth
 from logitfill_amd.packed import PackedKVManager
 from logitfill_amd.packed.reference import decode_into
+from tests.helpers import decode_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -79,6 +80,7 @@ def test_tiled_layouts(gpu, D, page, kg, vg, n_q, n_kv, lengths, q_len, dtype, p
     mgr, _, _, q, kn, vn = _setup(gpu, D, page, kg, vg, n_q, n_kv, lengths, q_len, dtype)
     want = _float64(mgr, q, kn, vn)
     tiled = _rel(_decode(mgr, q, kn, vn, _native.KERNEL_AUTO, pps), want)
+    assert decode_kernel(mgr) == _native.KERNEL_TILED
     plain = _rel(_decode(mgr, q, kn, vn, _native.KERNEL_VALU, pps), want)
     print(f"tiled {tiled:.2e} general {plain:.2e}")
     assert tiled < 2e-5 and tiled < 2 * plain + 1e-7
@@ -91,6 +93,30 @@ def test_tiled_single_tier(gpu, level):
     mgr, _, _, q, kn, vn = _setup(gpu, 64, 64, 32, 32, 6, 2, [5 * 64 + 3, 64], 1, torch.bfloat16, levels=levels)
     want = _float64(mgr, q, kn, vn)
     assert _rel(_decode(mgr, q, kn, vn, _native.KERNEL_AUTO), want) < 2e-5
+    assert decode_kernel(mgr) == _native.KERNEL_TILED
+
+
+@pytest.mark.parametrize("D,page,kg,vg,q_len,tail,new,offset", [
+    (64, 64, 32, 32, 1, torch.bfloat16, torch.float16, 0),
+    (64, 64, 64, 64, 7, torch.float32, torch.float16, 0),
+    (128, 128, 32, 32, 1, torch.float16, torch.float32, 0),
+    (128, 128, 128, 128, 5, torch.float32, torch.bfloat16, 0),  # the default layout, several tokens
+    (128, 64, 32, 64, 40, torch.bfloat16, torch.bfloat16, 1),   # new rows that start off 16 bytes
+    (256, 64, 64, 256, 1, torch.bfloat16, torch.float32, 0),
+    (256, 128, 64, 64, 6, torch.float16, torch.float16, 3),
+])
+def test_tiled_residual_rows_of_any_type(gpu, D, page, kg, vg, q_len, tail, new, offset):
+    """Residual pages and new tokens of unlike types, or rows off 16 bytes: element by element, with the
+    causal mask and, past the tail, rows that are clamped to stored ones."""
+    mgr, _, _, q, kn, vn = _setup(gpu, D, page, kg, vg, 8, 2, [3 * page + 17, 2 * page + 1, page], q_len, tail)
+    q = q.to(new)
+    kn, vn = (torch.zeros(t.numel() + offset, dtype=new, device=gpu)[offset:].view_as(t).copy_(t) for t in (kn, vn))
+    assert (kn.data_ptr() % 16 != 0) == (offset > 0)
+    want = _float64(mgr, q, kn, vn)
+    rel = _rel(_decode(mgr, q, kn, vn, _native.KERNEL_AUTO), want)
+    assert decode_kernel(mgr) == _native.KERNEL_TILED
+    print(f"rel {rel:.2e}")
+    assert rel < 2e-5
 
 
 def test_tiled_infinite_fp16_key(gpu):
@@ -107,6 +133,8 @@ def test_tiled_infinite_fp16_key(gpu):
     kn, vn = (torch.randn(1, 1, 1, 64, generator=g).to(gpu) for _ in range(2))
     a, b = (_decode(mgr, q, kn, vn, k) for k in (_native.KERNEL_AUTO, _native.KERNEL_VALU))
     assert torch.isfinite(a).all() and _rel(a, b) < 2e-5
+    _decode(mgr, q, kn, vn, _native.KERNEL_AUTO)
+    assert decode_kernel(mgr) == _native.KERNEL_TILED
 
 
 def test_general_kernel_group_of_one_and_a_half_chunks(gpu):
