@@ -306,7 +306,7 @@ def test_one_round_size(pages, n_kv, res, slots=512):
 
 def test_one_round_size_needs_a_clear_gain(slots=512):
     """A size past the even share is taken only where its estimate (largest item + overhead, one round)
-    beats the smaller sizes' by 7 %; drawn batches of both kinds occur."""
+    beats the smaller sizes' by 2 %; drawn batches of both kinds occur."""
     rng = np.random.default_rng(3)
     taken = declined = 0
     for _ in range(1500):
@@ -326,5 +326,5 @@ def test_one_round_size_needs_a_clear_gain(slots=512):
             return rounds * (max(-(-(p + 4) // k) for p, k in zip(pages, items)) + ITEM_OVERHEAD_PAGES), rounds
 
         taken += 1
-        assert cost(size)[1] == 1 and 1.07 * cost(size)[0] <= min(cost(s)[0] for s in range(1, even + 1))
+        assert cost(size)[1] == 1 and 1.02 * cost(size)[0] <= min(cost(s)[0] for s in range(1, even + 1))
     assert taken > 50 and declined > 50
