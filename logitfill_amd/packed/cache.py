@@ -19,6 +19,7 @@ batch != 1, ``cache.py:136-137``); ``commit`` then takes ``[batch, n_kv, T, D]``
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from typing import Optional
@@ -380,10 +381,14 @@ class _LayerStore:
             return
         segs = (ctypes.c_int32 * (4 * len(rows)))(*[x for row in rows for x in row])
         ks, vs = (ctypes.c_int64 * 3)(*key.stride()[:3]), (ctypes.c_int64 * 3)(*value.stride()[:3])
-        st = _native.load().lf_fill_tail(
-            tk.data_ptr(), tv.data_ptr(), key.data_ptr(), value.data_ptr(), _native.dtype_code(tk.dtype), ks, vs,
-            self.page_size, segs, len(rows), 1 if same else 0, self.batch, self.n_kv, self.head_dim,
-            _native.current_stream_ptr(self.device))
+        # (the default stream names no device: the launch needs the store's own to be current, as torch's copies
+        # see to by themselves)
+        here = torch.cuda.current_device() == self.device.index
+        with contextlib.nullcontext() if here else torch.cuda.device(self.device):
+            st = _native.load().lf_fill_tail(
+                tk.data_ptr(), tv.data_ptr(), key.data_ptr(), value.data_ptr(), _native.dtype_code(tk.dtype), ks, vs,
+                self.page_size, segs, len(rows), 1 if same else 0, self.batch, self.n_kv, self.head_dim,
+                _native.current_stream_ptr(self.device))
         _native.check(st, "lf_fill_tail")
 
     def _append_one(self, key: torch.Tensor, value: torch.Tensor) -> None:
