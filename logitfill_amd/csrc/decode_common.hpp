@@ -205,7 +205,9 @@ __device__ __forceinline__ void commit_new_rows(const DecodeParams& p, int b, in
 // is mostly empty (us per layer-step, decode_mfma / decode_rows, 28 q on 4 kv heads unless stated):
 // 28 rows x 125 pages 22.5 / 26.3, x 770 pages 74.1 / 73.4; 35 rows x 770 85.1 / 86.2; 56 rows x 125
 // (3 500) 38.2 / 30.6, x 770 110 / 91; 224 x 125 88 / 47; 64 rows, 2 kv heads, 124 pages (1 984) 23.1 /
-// 26.6; 120 rows, 2 kv heads, 28 pages (840) 19.2 / 21.4.
+// 26.6; 120 rows, 2 kv heads, 28 pages (840) 19.2 / 21.4.  4 620 drawn calls at or above the line: 0.84 to 11
+// times decode_mfma.hip's speed, 32 of them below 0.98 (up to five sequences, 41 to 72 rows, mostly below
+// 5 000 page-tiles; lines that leave those out lose as many gains of 1.1 to 1.5).
 constexpr int kRowsTiles = 6;
 constexpr int kRowsWork = 3000;
 

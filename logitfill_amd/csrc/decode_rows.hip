@@ -24,11 +24,13 @@
 // out of the sums again), so the sums carry no cancelling part.  The tail page and the new tokens
 // follow as dense chunks of 128 tokens through the same buffers.
 //
-// What bounds it: the LDS reads of the operands (12 of 1 KB per K-step and wave, 5 400 cycles of a
-// page's 15 200 for 128 rows) and the VALU work beside them (Qs 6.5 operations per slot and row, softmax
-// and P' split about 14 per score); the page's unpack takes 2 700.  512 new tokens x 28 q / 4 kv heads
-// over 16 384 tokens: 975 us a layer with decode_mfma.hip's 448 tiles of 8 rows, now 473 (470 before the
-// factor of Qs was the page's own).  Against float64 (float32 output) 0.2-1.1e-6, decode_mfma.hip 1-6e-5.
+// What bounds it: the LDS reads of the operands (12 of 1 KB per K-step and wave) and the VALU work
+// beside them (Qs 6.5 operations per slot and row, softmax and P' split about 14 per score).  Counters of 512
+// new tokens x 28 q / 4 kv heads over 16 384 tokens (224 workgroups of 64 pages, one per CU): a wave runs
+// 77 200 VALU operations, 11 400 products and 10 000 LDS instructions in 1.0 M cycles; over the chip the
+// VALU is 52 % and the matrix cores 30 % busy, and a cycle of LDS activity comes with 2.4 of bank conflicts.
+// The call takes 975 us a layer with decode_mfma.hip's 448 tiles of 8 rows, here 473 (470 before the factor
+// of Qs was the page's own).  Against float64 (float32 output) 0.2-1.1e-6, decode_mfma.hip 1-6e-5.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>

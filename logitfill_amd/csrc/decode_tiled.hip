@@ -31,10 +31,13 @@
 // a Value group go to its 16-channel tiles so that a lane's codes of one token lie in one or two
 // bytes of one word.
 //
-// What bounds it: per run of 64 tokens and wave, 2 000 VALU operations (unpacking codes, 1.5 each; the
-// three-part splits of Qs and P') and 150 products, of which a wave alone on its SIMD covers about
-// half; in short items the dependent loads before the first run (argument block, tier tables, q).
-// Measured with the general kernel before it (us per layer-step, decode and merge): 8 sequences of
+// What bounds it: VALU work (unpacking codes, 1.5 operations each; the three-part splits of Qs and P') at
+// one or two waves per SIMD, and in short items the dependent loads before the first run (argument block,
+// tier tables, q).  Counters of the two calls below: 5 700 VALU operations and 290 products per wave (two
+// runs of 64 tokens, prologue, residual, merge) at 38 % of the VALU and 8 % of the matrix cores busy;
+// 2 700 and 140 (one run) at 13 % and 3 %.  Registers: 256 VGPRs; head_dim 128 spills 9 to 28 of them, 256
+// (whose accumulators alone are 128) 72 to 322, and still takes 1 / 2.6 to 1 / 81 of the general kernel's
+// time (plan_tiled).  Measured with the general kernel before it (us per layer-step, decode and merge): 8 sequences of
 // 3K-8K tokens, 28 q / 4 kv heads, head_dim 128, Key and Value groups of 32 at Key 4.0 bits
 // 1 490 -> 35; 8 of 1.5K-5K, 14 / 2 heads, head_dim 64, 64-token pages and groups 124 -> 21.  Against
 // float64 (float32 output) 1.6e-6 and 1.5e-6 where the general kernel has 2.2e-6 and 2.0e-6.
@@ -883,7 +886,10 @@ __global__ __launch_bounds__(kThreads, 2) void decode_tiled_kernel(TiledParams t
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
-// LDS of a workgroup for this layer; false when the layout is outside this kernel.
+// LDS of a workgroup for this layer; false when the layout is outside this kernel.  Every layout inside goes to
+// it: 4 500 drawn calls (any page, Key and Value group, 1 to 16 sequences of 40 to 8 000 tokens, 1 to 17 new
+// tokens, all row types) take 1 / 2.0 to 1 / 43 of the general kernel's time at head_dim 64, 1 / 2.6 to 1 / 49
+// at 128 and 1 / 2.6 to 1 / 81 at 256.
 bool plan_tiled(const lf_packed_layer& L, TiledLayout& y) {
     const int D = L.head_dim;
     if (D != 64 && D != 128 && D != 256) return false;

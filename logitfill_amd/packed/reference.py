@@ -135,8 +135,8 @@ ALONE_FACTOR = 0.78
 
 # A size past the even share that makes one round is taken where its estimate is this much better than
 # the smaller items' rounds, and for one, two or four row tiles: 2 834 of 3 012 drawn batches with such a
-# size, 0.94 to 1.5 times the speed of the smaller items, median 1.14, seven below 0.98 (35 without the
-# margin).  Three and five tiles do not divide the 64 slots of an XCD, which the tiles of an (item, kv
+# size, 0.94 to 1.36 times the speed of the smaller items, median 1.14, seven below 0.98 (43 of 3 012
+# without the margin).  Three and five tiles do not divide the 64 slots of an XCD, which the tiles of an (item, kv
 # head) share (decode_mfma.hip): 760 batches 0.63 to 1.5 times, median 0.83 where an XCD gets a 65th
 # workgroup.
 ONE_ROUND_GAIN = 1.02
