@@ -572,7 +572,6 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
     kernel = kernel_choice() if kernel is None else kernel
     lib = _native.load()
     P = layer.page_size
-    hist_pages = tuple(h // P for h in layer.hist_lens)
     tail_k, tail_v = layer.tail_buffers()
     if key_new is not None and value_new.dtype != key_new.dtype:
         raise TypeError("key_new and value_new must share a dtype")
@@ -580,14 +579,15 @@ def decode_into(manager, layer_idx: int, query: torch.Tensor, key_new, value_new
     if key_new is not None:
         k_ptr, v_ptr = key_new.data_ptr(), value_new.data_ptr()
     # which kernel takes the call, and so how its plan is sized: asked again when something it
-    # depends on changes
-    rule_key = (hist_pages, q_len, kernel, query.dtype, None if key_new is None else key_new.dtype,
+    # depends on changes (the lengths are compared as they are, the pages counted then)
+    rule_key = (tuple(layer.hist_lens), q_len, kernel, query.dtype, None if key_new is None else key_new.dtype,
                 None if tail_k is None else tail_k.dtype, (q_ptr & 15) << 8 | (k_ptr & 15) << 4 | v_ptr & 15)
     cached_rule = layer.__dict__.get("_lf_plan_rule")
     if cached_rule is None or cached_rule[0] != rule_key:
-        cached_rule = (rule_key, plan_rule(manager, layer, rule_key, q_ptr, k_ptr, v_ptr))
+        hist_pages = tuple(h // P for h in rule_key[0])
+        cached_rule = (rule_key, plan_rule(manager, layer, (hist_pages, *rule_key[1:]), q_ptr, k_ptr, v_ptr), hist_pages)
         layer.__dict__["_lf_plan_rule"] = cached_rule
-    rule = cached_rule[1]
+    _, rule, hist_pages = cached_rule
     res_pages = rule.residual(max(layer.tail_lens), q_len)
     if pages_per_split is None:
         # the split depends on the history, the kernel, the residual cost and the environment's
